@@ -338,7 +338,9 @@ int long_ray_of(const mexct_opts* o) {
   return o->long_ray < 0 ? INT_MAX : o->long_ray;
 }
 
-// z-fastest FP volume layout for storage st (see fpz.hip): DUAL for f32,
+// z-fastest FP volume layout for storage st.  Parallel and fan rays, which
+// stay in a plane of voxel centres, take the column projector (COL,
+// fpc.hip) while its copy stays below 4 GiB.  Else (see fpz.hip) DUAL for f32,
 // QUAD for 2-byte storage while the copy stays below 4 GiB (32-bit buffer
 // offsets); past that the same copies read through 64-bit addresses
 // (DUAL64 / QUAD64, below 2^32 elements); else -1 (the x-fastest
@@ -347,11 +349,13 @@ int long_ray_of(const mexct_opts* o) {
 // MEXCT_FP_LAYOUT=wide64 takes the 64-bit forms below 4 GiB as well, and
 // MEXCT_FP_LAYOUT=plain the one-value-per-element copy (below 2 GiB), so
 // that every address path can be compared with the default on one volume.
-int fp_layout(int64_t W, int64_t H, int st, size_t* bytes) {
+int fp_layout(int geom, int64_t W, int64_t H, int st, size_t* bytes) {
   const size_t es = (size_t)store_bytes(st);
   // the z-fastest projector's 24-bit index multiplies need (W+4)(H+4) < 2^23
   if ((W + 4) * (H + 4) >= ((int64_t)1 << 23)) return -1;
   const char* force = getenv("MEXCT_FP_LAYOUT");
+  if (!force && (geom == GEOM_PAR || geom == GEOM_FAN) && fpc_shape(W, H, st, bytes))
+    return LAYOUT_COL;
   if (force && !strcmp(force, "plain")) {
     *bytes = (size_t)(W + 4) * (W + 4) * (H + 4) * es;
     return *bytes < ((size_t)1 << 31) ? LAYOUT_PLAIN : -1;
@@ -370,6 +374,9 @@ hipError_t build_fp_volume(int layout, const void* in, int in_dt, int64_t sy, in
                            void* out, int st, int64_t W, int64_t H, int mode, hipStream_t s,
                            const uint32_t* scale) {
   layout = base_layout(layout);  // the 64-bit layouts hold the same copies
+  if (layout == LAYOUT_COL)
+    return launch_pad3c(in, in_dt, sy, sz, out, st, (int)W, (int)W, (int)H, fpc_rows(H, st), mode, s,
+                        scale);
   if (layout == LAYOUT_DUAL)
     return launch_pad3d(in, in_dt, sy, sz, out, st, (int)W, (int)W, (int)H, mode, s, scale);
   if (layout == LAYOUT_QUAD)
@@ -638,7 +645,7 @@ size_t op_workspace_bytes(int op, int geom, int st, int64_t W, int64_t H, int64_
   size_t b = common;
   if (op == MEXCT_OP_FP) {
     size_t lbytes = 0;
-    const int layout = fp_layout(W, H, st, &lbytes);
+    const int layout = fp_layout(geom, W, H, st, &lbytes);
     b += layout >= 0 ? slot(lbytes * nitems) : slot((size_t)(W + 4) * (W + 4) * (H + 4) * es);
     return b;
   }
@@ -673,7 +680,7 @@ size_t op_workspace_bytes(int op, int geom, int st, int64_t W, int64_t H, int64_
   const size_t pv = (size_t)2 * (W + 4) * (H + 3);
   const size_t pbytes = (pv * cmax * es + 3) / 4 * 4;
   size_t lbytes = 0;
-  (void)fp_layout(W, H, st, &lbytes);
+  (void)fp_layout(geom, W, H, st, &lbytes);
   b += 6 * slot(psz) + 2 * slot(padsz) + 2 * slot(vsz) +
        slot(tv_partials_count((int)W, (int)W, (int)H) * 8) + slot(256) + 2 * slot(pbytes) +
        slot(lbytes);
@@ -747,7 +754,7 @@ int fp_run(mexct_ctx* c, const void* vol, int32_t vol_dtype, int items, int64_t 
   void* pad;
   const size_t pbytes = (size_t)(W + 4) * (W + 4) * (H + 4) * store_bytes(st);
   size_t lbytes = 0;
-  const int layout = fp_layout(W, H, st, &lbytes);
+  const int layout = fp_layout(geom, W, H, st, &lbytes);
   const float2* sc;
   const size_t vel = (size_t)W * W * H;  // elements of one input volume
   if (loads_only && (layout < 0 || wide64(layout)))
@@ -783,6 +790,9 @@ int fp_run(mexct_ctx* c, const void* vol, int32_t vol_dtype, int items, int64_t 
     z.out_stride = (uint64_t)W * H * nProj;
     RC(upload_ptrs(c, out_ptrs, items, &z.outs));
     z.loads_only = loads_only;
+    auto launch = [&](const FPZLaunch& l) {
+      return layout == LAYOUT_COL ? launch_fpc(l, c->stream) : launch_fpz(l, c->stream);
+    };
     const TuneKey key{MEXCT_OP_FP, geom, st, W, H, nProj};
     TuneVal tv;
     if (tune_find(key, &tv)) {
@@ -793,7 +803,7 @@ int fp_run(mexct_ctx* c, const void* vol, int32_t vol_dtype, int items, int64_t 
         FPZLaunch t = z;
         t.vchunk_log2 = cand[i];
         t.nviews = std::min<int>(nProj, kTuneViewsFP);
-        HIPCHK(launch_fpz(t, c->stream));
+        HIPCHK(launch(t));
         return MEXCT_OK;
       }, &tv.ms);
       if (best < 0) return best;
@@ -801,7 +811,7 @@ int fp_run(mexct_ctx* c, const void* vol, int32_t vol_dtype, int items, int64_t 
       tune_store(key, tv);
       z.vchunk_log2 = tv.a;
     }
-    HIPCHK(launch_fpz(z, c->stream));
+    HIPCHK(launch(z));
     return MEXCT_OK;
   }
   if (items != 1) return fail(MEXCT_ENOTSUP, "volume too large to batch");
@@ -1108,7 +1118,7 @@ int mexct_g3d_fp_dev(mexct_ctx* c, const void* vol, int32_t vol_dtype, int64_t s
   void* pad;
   const float2* sc;
   size_t lbytes = 0;
-  const int layout = fp_layout(side, nSlices, st, &lbytes);
+  const int layout = fp_layout(GEOM_G3D, side, nSlices, st, &lbytes);
   if (layout >= 0) {
     // z-fastest volume as for the standard geometries; a wave marches 64
     // consecutive detector rows of one column, whose rays are near each
@@ -1313,7 +1323,7 @@ int osc_subsets(mexct_ctx* c, float* mu_pad, int W, int H, float* pre, float* po
   void* mz;
   const int64_t MPX = W + 4, MPXY = (int64_t)(W + 4) * (W + 4);
   size_t lbytes = 0;
-  const int layout = fp_layout(W, H, st, &lbytes);
+  const int layout = fp_layout(geom, W, H, st, &lbytes);
   if (layout < 0)
     return fail(MEXCT_EINVAL,
                 "OSC: the projected volume copy needs (W+4)*(H+4) = %lld below 2^23 and fewer "
@@ -1348,7 +1358,7 @@ int osc_subsets(mexct_ctx* c, float* mu_pad, int W, int H, float* pre, float* po
       f.stride = numSubsets;
       f.count = count;
       f.sad = sad;
-      HIPCHK(launch_osc_fp(f, c->stream));
+      HIPCHK(layout == LAYOUT_COL ? launch_osc_fpc(f, c->stream) : launch_osc_fp(f, c->stream));
     }
     OSCBPLaunch b;
     b.pre_pad = pp;

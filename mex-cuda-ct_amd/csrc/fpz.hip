@@ -45,8 +45,6 @@ namespace mexct {
 // f32 104.6 -> 97.8 ms, f16 99.4 -> 90.8 ms with 1, 104.0 / 117.6 / 106.2 ms
 // f32 with 2 / 4 / 8)
 constexpr uint32_t kViewChunkLog2 = 3, kViewChunkLog2G3D = 4, kViewChunkLog2Osc = 0;
-// default ray length (samples) above which 2-byte ray sums are compensated
-constexpr int kLongRay = 1024;
 
 struct FPZArgs {
   const void* vol;     // z-fastest haloed volume
@@ -497,28 +495,6 @@ __device__ __forceinline__ float march_z(__amdgpu_buffer_rsrc_t r, const FPZArgs
   }
   return march_loopd<S, STEP2, LAYOUT, true, fetch_ahead<S, EPI>(), loads_only(EPI)>(
       r, a, cur, inc, n, fnx, fny, fnz, base, vb);
-}
-
-// Storage of the OSC ratio terms for a volume storage S.  They span the
-// counts times the line integral (up to ~1e5 and down to ~1e-5 and below),
-// beyond FP16's range, so an FP16 volume copy pairs with BF16 ratio terms.
-template <typename S>
-struct OscPad {
-  typedef S T;
-};
-template <>
-struct OscPad<_Float16> {
-  typedef bf16_t T;
-};
-
-// Value v of detector pixel (u, row) into a row-paired copy: pair q (that
-// of (u, row)) holds it first, the pair of (u, row - 1) second.
-template <typename P>
-__device__ __forceinline__ void osc_pair_store(void* pad, size_t q, int PW, float v) {
-  P* p = (P*)pad;
-  const P s = Store<P>::from(v);
-  p[2 * q] = s;
-  p[2 * (q - (size_t)PW) + 1] = s;
 }
 
 // EPI 0: store the ray sum.  EPI 1: OSC ratio terms of CUDAmex_oscIter.cu:262-268

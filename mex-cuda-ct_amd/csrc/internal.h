@@ -33,6 +33,14 @@ hipError_t launch_pad3d(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
 hipError_t launch_pad3q(const void* in, int in_dt, int64_t in_sy, int64_t in_sz, void* out,
                         int st_dt, int nx, int ny, int nz, int mode, hipStream_t st,
                         const uint32_t* scale_max = nullptr);
+// Copy for the column projector (fpc.hip): z-fastest with a 2-texel halo in x
+// and y only and pz >= nz rows per voxel column (fpc_rows).  f32: V(x,y,z) at
+// ((x+2)*(ny+4) + y+2)*pz + z; 2-byte storage: the quads of launch_pad3q at
+// ((x+2)*(ny+3) + y+2)*pz + z.  An element is NaN where it or the one at z+1
+// holds a value that is not finite.
+hipError_t launch_pad3c(const void* in, int in_dt, int64_t in_sy, int64_t in_sz, void* out,
+                        int st_dt, int nx, int ny, int nz, int pz, int mode, hipStream_t st,
+                        const uint32_t* scale_max = nullptr);
 // 2D stack, row-grouped: in [w,h,n] -> out [rows, w+4, h+2*zh-1, n] where
 // element (px, py) holds the haloed values at rows py-zh .. py-zh+rows-1 of
 // column px (rows = 2, or 4 for 2-byte storage; zh >= 2 rows of halo).
@@ -66,7 +74,15 @@ hipError_t launch_fp(const FPLaunch& a, hipStream_t st);
 // z-fastest volume layouts of the standard-geometry FP (see fpz.hip)
 // DUAL64 / QUAD64: the DUAL / QUAD copies past 4 GiB, read with 64-bit
 // addresses instead of 32-bit buffer offsets (every index clamped)
-enum { LAYOUT_PLAIN = 0, LAYOUT_QUAD = 1, LAYOUT_DUAL = 2, LAYOUT_DUAL64 = 3, LAYOUT_QUAD64 = 4 };
+// COL: the column projector's copy (fpc.hip)
+enum {
+  LAYOUT_PLAIN = 0,
+  LAYOUT_QUAD = 1,
+  LAYOUT_DUAL = 2,
+  LAYOUT_DUAL64 = 3,
+  LAYOUT_QUAD64 = 4,
+  LAYOUT_COL = 5
+};
 constexpr int base_layout(int l) {
   return l == LAYOUT_DUAL64 ? LAYOUT_DUAL : l == LAYOUT_QUAD64 ? LAYOUT_QUAD : l;
 }
@@ -97,6 +113,14 @@ struct FPZLaunch {
 };
 hipError_t launch_fpz(const FPZLaunch& a, hipStream_t st);
 
+// Column projector (fpc.hip): par and fan on a launch_pad3c copy of
+// fpc_shape bytes; false where the copy would pass 4 GiB or its rows the
+// 24-bit index multiplies.  The same arguments and bits as launch_fpz
+// (layout unused).
+bool fpc_shape(int64_t W, int64_t H, int st_dt, size_t* bytes);
+int fpc_rows(int64_t H, int st_dt);
+hipError_t launch_fpc(const FPZLaunch& a, hipStream_t st);
+
 // OSC forward projection + ratio terms over the views first, first+stride, ...
 struct OSCFPLaunch {
   const void* mu_z;     // z-fastest volume of storage st_dt with a zero (border) halo
@@ -113,6 +137,8 @@ struct OSCFPLaunch {
   int long_ray = 0;  // as FPZLaunch::long_ray
 };
 hipError_t launch_osc_fp(const OSCFPLaunch& a, hipStream_t st);
+// the same by the column projector (par and fan, mu_z a launch_pad3c copy)
+hipError_t launch_osc_fpc(const OSCFPLaunch& a, hipStream_t st);
 
 // ---- backprojection (bp.hip)
 struct BPLaunch {

@@ -194,17 +194,23 @@ template <>
 struct Quad<_Float16> {
   typedef _Float16 v4 __attribute__((ext_vector_type(4)));
   __device__ static void put(_Float16* out, size_t e, float a, float b, float c, float d) {
+    *(uint64_t*)(out + 4 * e) = bits(a, b, c, d);
+  }
+  __device__ static uint64_t bits(float a, float b, float c, float d) {
     const float dx = c - a;
     v4 q = {(_Float16)a, (_Float16)(b - a), (_Float16)dx, (_Float16)((d - b) - dx)};
-    *(v4*)(out + 4 * e) = q;
+    return __builtin_bit_cast(uint64_t, q);
   }
 };
 template <>
 struct Quad<bf16_t> {
   typedef uint16_t v4 __attribute__((ext_vector_type(4)));
   __device__ static void put(bf16_t* out, size_t e, float a, float b, float c, float d) {
+    *(uint64_t*)(out + 4 * e) = bits(a, b, c, d);
+  }
+  __device__ static uint64_t bits(float a, float b, float c, float d) {
     v4 q = {f32_to_bf16(a), f32_to_bf16(b), f32_to_bf16(c), f32_to_bf16(d)};
-    *(v4*)(out + 4 * e) = q;
+    return __builtin_bit_cast(uint64_t, q);
   }
 };
 
@@ -241,6 +247,70 @@ __global__ __launch_bounds__(256) void pad3q_kernel(const void* __restrict__ in,
     if (qx < QX && qz < QZ)
       Quad<S>::put(out, ((size_t)qx * QY + qy) * QZ + qz, tile[0][tz][lx], tile[1][tz][lx],
                    tile[0][tz][lx + 1], tile[1][tz][lx + 1]);
+  }
+}
+
+// Copy for the column projector (see launch_pad3c): z-fastest, two texels of
+// halo in x and y, none in z, pz >= nz rows per column.  A block
+// covers 32 z x 32 x of one y; the (z .. z+32, x .. x+32) tiles of input row
+// y (and y + 1 for the quads) are staged in LDS.  A value is stored as NaN
+// where it or the one at z + 1 is not finite (what the weight-0 z lerp makes
+// of them).
+__device__ __forceinline__ bool finite_bits(uint32_t expo, uint32_t mask) {
+  return (expo & mask) != mask;
+}
+template <typename S>
+__device__ __forceinline__ bool quad_finite(uint64_t q) {
+  constexpr uint32_t m = __is_same(S, _Float16) ? 0x7c00u : 0x7f80u;
+  return finite_bits((uint32_t)q, m) && finite_bits((uint32_t)(q >> 16), m) &&
+         finite_bits((uint32_t)(q >> 32), m) && finite_bits((uint32_t)(q >> 48), m);
+}
+
+template <typename S>
+__global__ __launch_bounds__(256) void pad3c_kernel(const void* __restrict__ in, int in_dt,
+                                                    int64_t in_sy, int64_t in_sz,
+                                                    S* __restrict__ out, int nx, int ny, int nz,
+                                                    int pz, int mode, const uint32_t* scale_max) {
+  constexpr bool Q = sizeof(S) == 2;  // corner quads
+  constexpr int TY = Q ? 2 : 1, LX = 32 + (Q ? 1 : 0);
+  __shared__ float tile[TY][33][34];
+  const int sexp = pow2_exp(scale_max);
+  const int DX = nx + 2 * HALO - (Q ? 1 : 0), DY = ny + 2 * HALO - (Q ? 1 : 0);
+  const int z0 = blockIdx.x * 32, dx0 = blockIdx.y * 32, dy = blockIdx.z;
+  for (int e = threadIdx.x; e < TY * 33 * LX; e += 256) {
+    const int r = e / (33 * LX);
+    const int rem = e - r * (33 * LX);
+    const int lz = rem / LX, lx = rem - lz * LX;
+    int i = dx0 + lx - HALO, j = dy + r - HALO, k = z0 + lz;
+    float v = 0.f;
+    if (mode == ADDR_CLAMP) {
+      i = clampi(i, 0, nx - 1);
+      j = clampi(j, 0, ny - 1);
+      k = clampi(k, 0, nz - 1);
+      v = load_any(in, in_dt, (size_t)i + (size_t)in_sy * j + (size_t)in_sz * k);
+    } else if (i >= 0 && i < nx && j >= 0 && j < ny && k < nz) {
+      v = load_any(in, in_dt, (size_t)i + (size_t)in_sy * j + (size_t)in_sz * k);
+    }
+    tile[r][lz][lx] = ldexpf(v, -sexp);
+  }
+  __syncthreads();
+  const int tz = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
+  for (int p = 0; p < 4; ++p) {
+    const int lx = ty + 8 * p;
+    const int dx = dx0 + lx, z = z0 + tz;
+    if (dx >= DX || z >= pz) continue;
+    const size_t e = ((size_t)dx * DY + dy) * pz + z;
+    if constexpr (Q) {
+      uint64_t q = Quad<S>::bits(tile[0][tz][lx], tile[1][tz][lx], tile[0][tz][lx + 1],
+                                tile[1][tz][lx + 1]);
+      const uint64_t n = Quad<S>::bits(tile[0][tz + 1][lx], tile[1][tz + 1][lx],
+                                      tile[0][tz + 1][lx + 1], tile[1][tz + 1][lx + 1]);
+      if (!quad_finite<S>(q) || !quad_finite<S>(n)) q = ~0ull;
+      *(uint64_t*)(out + 4 * e) = q;
+    } else {
+      const float v = tile[0][tz][lx], n = tile[0][tz + 1][lx];
+      out[e] = __builtin_isfinite(v) && __builtin_isfinite(n) ? v : __builtin_nanf("");
+    }
   }
 }
 
@@ -334,6 +404,23 @@ hipError_t launch_pad3q(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
                                               mode, scale_max);
   else
     pad3q_kernel<bf16_t><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (bf16_t*)out, nx, ny, nz,
+                                            mode, scale_max);
+  return hipGetLastError();
+}
+
+hipError_t launch_pad3c(const void* in, int in_dt, int64_t in_sy, int64_t in_sz, void* out,
+                        int st_dt, int nx, int ny, int nz, int pz, int mode, hipStream_t st,
+                        const uint32_t* scale_max) {
+  const dim3 g((unsigned)((pz + 31) / 32), (unsigned)((nx + 2 * HALO + 31) / 32),
+               (unsigned)(ny + 2 * HALO - (st_dt == 0 ? 0 : 1)));
+  if (st_dt == 0)
+    pad3c_kernel<float><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (float*)out, nx, ny, nz, pz,
+                                           mode, scale_max);
+  else if (st_dt == 1)
+    pad3c_kernel<_Float16><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (_Float16*)out, nx, ny, nz,
+                                              pz, mode, scale_max);
+  else
+    pad3c_kernel<bf16_t><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (bf16_t*)out, nx, ny, nz, pz,
                                             mode, scale_max);
   return hipGetLastError();
 }

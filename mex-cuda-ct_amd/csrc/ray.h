@@ -118,4 +118,29 @@ __device__ __forceinline__ int clip_ray(const R3& st, const R3& en, float bx, fl
   return q < (float)kMaxSamples ? (int)q : kMaxSamples;
 }
 
+// default ray length (samples) above which 2-byte ray sums are compensated
+constexpr int kLongRay = 1024;
+
+// Storage of the OSC ratio terms for a volume storage S.  They span the
+// counts times the line integral (up to ~1e5 and down to ~1e-5 and below),
+// beyond FP16's range, so an FP16 volume copy pairs with BF16 ratio terms.
+template <typename S>
+struct OscPad {
+  typedef S T;
+};
+template <>
+struct OscPad<_Float16> {
+  typedef bf16_t T;
+};
+
+// Value v of detector pixel (u, row) into a row-paired copy: pair q (that
+// of (u, row)) holds it first, the pair of (u, row - 1) second.
+template <typename P>
+__device__ __forceinline__ void osc_pair_store(void* pad, size_t q, int PW, float v) {
+  P* p = (P*)pad;
+  const P s = Store<P>::from(v);
+  p[2 * q] = s;
+  p[2 * (q - (size_t)PW) + 1] = s;
+}
+
 }  // namespace mexct
