@@ -654,7 +654,9 @@ size_t op_workspace_bytes(int op, int geom, int st, int64_t W, int64_t H, int64_
     const int rows = st != MEXCT_F32 && (geom != 2 || (double)sad > 2.02 * hw) ? 4 : 2;
     bool zc;
     const int zh = bp_row_halo(W, H, geom, sad, rows, st, &zc);
-    b += slot((size_t)(W + 4) * (H + 2 * zh - 1) * rows * es * n * nitems);
+    size_t vb = (size_t)(W + 4) * (H + 2 * zh - 1) * rows * es;
+    (void)bpc_shape(W, H, geom, sad, st, nullptr, &vb);
+    b += slot(vb * n * nitems);
     if (geom == 2 && st == MEXCT_F32) {
       size_t cfv = 0;  // the largest chain of any tuning candidate
       for (int sup : {2, 4, 8})
@@ -914,10 +916,12 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
   const int rows = st != MEXCT_F32 && (geom != 2 || (double)sad > 2.02 * hw) ? 4 : 2;
   bool zclamp;
   const int zh = bp_row_halo(W, H, geom, sad, rows, st, &zclamp);
-  const size_t rp_bytes = (size_t)(W + 4) * (H + 2 * zh - 1) * rows * store_bytes(st);
+  size_t rp_bytes = (size_t)(W + 4) * (H + 2 * zh - 1) * rows * store_bytes(st);
   if ((double)rp_bytes >= 2147483648.0)
     return fail(MEXCT_EINVAL, "detector too large (%lld x %lld)", (long long)W, (long long)H);
   if ((double)W * W * H >= 4294967296.0) return fail(MEXCT_EINVAL, "volume too large");
+  // par and fan: by detector columns, on a copy of single rows
+  const bool col = bpc_shape(W, H, geom, sad, st, nullptr, &rp_bytes);
   DevGuard g(c->device);
   void* pad;
   const size_t sino_stride = rp_bytes * (size_t)std::max<int64_t>(nProj, 1);
@@ -928,11 +932,15 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
     RC(max_bits(c, (const float*)sino, sel, kSlotSino, &smax, items, sel, in_ptrs));
   const size_t in_es = (size_t)store_bytes(sino_dtype);
   if (nProj > 0)
-    for (int i = 0; i < items; ++i)
-      HIPCHK(launch_pad2(in_ptrs ? in_ptrs[i] : (const char*)sino + i * sel * in_es, sino_dtype,
-                         (char*)pad + i * sino_stride,
-                         st, (int)W, (int)H, (int)nProj, ADDR_CLAMP, c->stream,
-                         smax ? smax + i : nullptr, rows, zh));
+    for (int i = 0; i < items; ++i) {
+      const void* in = in_ptrs ? in_ptrs[i] : (const char*)sino + i * sel * in_es;
+      const uint32_t* m = smax ? smax + i : nullptr;
+      void* o = (char*)pad + i * sino_stride;
+      HIPCHK(col ? launch_pad2c(in, sino_dtype, o, st, (int)W, (int)H, (int)nProj,
+                                bpc_rows(H, st), c->stream, m)
+                 : launch_pad2(in, sino_dtype, o, st, (int)W, (int)H, (int)nProj, ADDR_CLAMP,
+                               c->stream, m, rows, zh));
+    }
   const float2* sc = nullptr;
   RC(c->sincos_table(angles, (int)nProj, &sc));
   BPLaunch a;
@@ -1004,7 +1012,7 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
       t.super_ = cand[i].first;
       t.zr = cand[i].second;
       t.nviews = (int)std::min<int64_t>(nProj, kTuneViews);
-      HIPCHK(launch_bp(t, c->stream));
+      HIPCHK(col ? launch_bpc(t, c->stream) : launch_bp(t, c->stream));
       return MEXCT_OK;
     }, &tv.ms);
     if (best < 0) return best;
@@ -1014,7 +1022,7 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
     a.super_ = tv.a;
     if (zr_free) a.zr = tv.b;
   }
-  HIPCHK(launch_bp(a, c->stream));
+  HIPCHK(col ? launch_bpc(a, c->stream) : launch_bp(a, c->stream));
   return MEXCT_OK;
 }
 }  // namespace

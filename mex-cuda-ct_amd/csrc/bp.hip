@@ -1,5 +1,6 @@
-// bp.hip -- voxel-driven backprojectors (standard geometries and the OSC
-// dual backprojection with its update) and the general-3D ray-driven
+// bp.hip -- voxel-driven backprojectors (cone, fan with the source near the
+// circle, and the OSC dual backprojection with its update; parallel and other
+// fan scans take the column kernel, bpc.hip) and the general-3D ray-driven
 // scatter, for gfx950.
 //
 // Voxel-driven BP (CUDAmex_BP.cu:44-221): the reference launches one kernel
@@ -11,7 +12,7 @@
 // order, starting from 0, so the float sum is the reference's sum.
 //
 // The reference steps the detector row by a running float sum,
-// proj_z += U per slice (CUDAmex_BP.cu:208-219).  For par and fan the
+// proj_z += U per slice (CUDAmex_BP.cu:208-219).  For fan the
 // running sum holds k + 0.5 exactly and is computed directly; for cone the
 // thread replays the z0 additions that precede its first voxel, so every
 // sample lands exactly where the reference's sample lands.
@@ -101,12 +102,7 @@ __device__ __forceinline__ void bp_view_geom(float x, float y, float sB, float c
                                              float& pz, float& dz) {
   float s = x * cB + y * sB;
   float t = -x * sB + y * cB;
-  if (GEOM == GEOM_PAR) {  // CUDAmex_BP.cu:92-95
-    U = 1.f;
-    py = t * U + (float)hw + 1.f;
-    pz = -v0 * U + v0 + 0.5f;
-    dz = U;
-  } else if (GEOM == GEOM_FAN) {  // :149-154
+  if (GEOM == GEOM_FAN) {  // CUDAmex_BP.cu:149-154
     U = SR / (SR - s);
     py = t * U + (float)hw + 1.f;
     pz = 0.5f;
@@ -421,7 +417,6 @@ static void bp_dispatch_g(const BPKArgs& k0, int geom, hipStream_t st) {
     return;
   }
   switch (geom) {
-    case GEOM_PAR: bp_kernel<GEOM_PAR, ZR, S, SMALL, RQ, ZC><<<g, 64, 0, st>>>(k); break;
     case GEOM_FAN: bp_kernel<GEOM_FAN, ZR, S, SMALL, RQ, ZC><<<g, 64, 0, st>>>(k); break;
     default: bp_kernel<GEOM_CONE, ZR, S, SMALL, RQ, ZC><<<g, 64, 0, st>>>(k); break;
   }
@@ -497,6 +492,7 @@ hipError_t launch_bp(const BPLaunch& a, hipStream_t st) {
   k.outs = a.outs;
   k.loads_only = a.loads_only ? 1 : 0;
   if (a.loads_only && a.geom != GEOM_CONE) return hipErrorInvalidValue;
+  if (a.geom == GEOM_PAR) return hipErrorInvalidValue;  // bpc.hip takes every one
   if (k.n_logical == 0) return hipSuccess;
   const size_t view_bytes = (size_t)k.PV * es2;
   int chunk = (int)std::max<size_t>(1, (((size_t)1 << 31) - 1) / view_bytes);

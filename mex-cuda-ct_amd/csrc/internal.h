@@ -47,6 +47,11 @@ hipError_t launch_pad3c(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
 hipError_t launch_pad2(const void* in, int in_dt, void* out, int st_dt, int w, int h, int n,
                        int mode, hipStream_t st, const uint32_t* scale_max = nullptr,
                        int rows = 2, int zh = 2);
+// Sinogram copy for the column backprojector (bpc.hip): in [w,h,n] ->
+// out[(view*(w+4) + u+2)*pv + v], pv >= h rows per detector column (bpc_rows).
+// A value is NaN where it or the one at v+1 is not finite.
+hipError_t launch_pad2c(const void* in, int in_dt, void* out, int st_dt, int w, int h, int n, int pv,
+                        hipStream_t st, const uint32_t* scale_max = nullptr);
 // scale_max (pad3z, pad3q, pad2): when non-null, the bits of max|in|; the
 // copy holds in * 2^-pow2_exp(scale_max) (see common.h).
 // 3D interior copy between a padded f32 volume and a plain one.
@@ -171,6 +176,12 @@ struct BPLaunch {
 // floats of BP chain scratch per view (cone f32, z-range zr, super-tile side)
 size_t bp_chain_floats_per_view(int W, int H, int zr, int super_);
 hipError_t launch_bp(const BPLaunch& a, hipStream_t st);
+// Column backprojector (bpc.hip): par and fan on a launch_pad2c copy of
+// view_bytes per view; false for shapes it does not take.  The same
+// arguments and bits as launch_bp (zr, rows, chain, zh, zclamp unused).
+bool bpc_shape(int64_t W, int64_t H, int geom, float sad, int st_dt, int* cw, size_t* view_bytes);
+int bpc_rows(int64_t H, int st_dt);
+hipError_t launch_bpc(const BPLaunch& a, hipStream_t st);
 
 struct OSCBPLaunch {
   const void* pre_pad;    // [2, W+4, H+3, count] of storage st_dt (F32 or BF16)

@@ -116,3 +116,64 @@ def test_column_fp_compensated_sums_equal_ray_fp(gpu, monkeypatch, st):
         out.append(o.cpu().numpy())
     ctx.close()
     assert np.array_equal(out[0], out[1])
+
+
+# slices: one, a lane's 4 (8) and its neighbours, around a workgroup's 16..128;
+# columns: odd, around tiles of 8, the smallest circle; views: around the four
+# of a stage; sizes past the 2048 workgroups from which it takes 64 (128)
+BP_SIZES = [(1, 5, 2), (3, 2, 3), (4, 1, 1), (9, 3, 5), (16, 16, 4), (33, 17, 7), (40, 65, 3), (23, 130, 9),
+            (200, 131, 6), (370, 3, 2)]
+
+
+@pytest.mark.parametrize("bad", [False, True])
+@pytest.mark.parametrize("W,H,n", BP_SIZES)
+def test_column_bp_equals_oracle(gpu, W, H, n, bad):
+    import torch
+
+    import oracle as O
+    ctx = device.Context(0)
+    ang = (np.arange(n) * (2 * np.pi / n) + 0.03).astype(np.float32)
+    p = _rng(W + H).uniform(-1, 1, (n, H, W)).astype(np.float32)
+    if bad:
+        p = _spoil(p, W)
+    sino = torch.from_numpy(p).cuda()
+    r = W // 2
+    # the fan sources: one whose tiles reach many detector columns, a usual
+    # one, and one within 20% of the circle (the general kernel)
+    for geom, sad in ((0, 300.0), (1, 1.9 * r + 1), (1, 900.0), (1, 1.15 * r + 0.1)):
+        want = np.ascontiguousarray(O.bp(np.asfortranarray(p.transpose(2, 1, 0)), sad, ang,
+                                         geom).transpose(2, 1, 0))
+        nan = np.isnan(want)
+        for st in STORAGES:
+            print(f"bp geom={geom} sad={sad} storage={st} W={W} H={H} n={n} bad={bad}", flush=True)
+            got = torch.full((H, W, W), -7.0, device="cuda")
+            ctx.bp(sino, sad, ang, geom, got, storage=st)
+            g = got.cpu().numpy()
+            if st == mexct.F32:
+                assert np.array_equal(g, want, equal_nan=True), (geom, sad)
+                continue
+            assert np.array_equal(np.isnan(g), nan), (geom, sad, st)
+            # a value's error: its storage rounding (2^-11, 2^-8 of max|P| = 1)
+            # and, f16, two packed roundings of the column lerp, times the
+            # distance weight, per view
+            u = 1.0 if geom == 0 else sad / (sad - r)
+            tol = n * u * u * (4 * 2.0 ** -11 if st == mexct.F16 else 1.1 * 2.0 ** -8)
+            assert np.abs(g - want)[~nan].max(initial=0.0) <= tol, (geom, sad, st)
+    ctx.close()
+
+
+def test_column_bp_batch_equals_single(gpu):
+    import torch
+    ctx = device.Context(0)
+    G, W, H, n = 3, 57, 21, 10
+    ang = (np.arange(n) * 0.4).astype(np.float32)
+    sinos = torch.from_numpy(_rng(5).uniform(-1, 1, (G, n, H, W)).astype(np.float32)).cuda()
+    for geom in (0, 1):
+        for st in STORAGES:
+            a = torch.full((G, H, W, W), -7.0, device="cuda")
+            ctx.bp_batch(sinos, 400.0, ang, geom, a, storage=st)
+            for i in range(G):
+                b = torch.full((H, W, W), -9.0, device="cuda")
+                ctx.bp(sinos[i], 400.0, ang, geom, b, storage=st)
+                assert torch.equal(a[i], b)
+    ctx.close()
