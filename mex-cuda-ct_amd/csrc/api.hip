@@ -74,6 +74,8 @@ enum Slot {
   WS_MUPAD,
   WS_MUOLD,
   WS_TVG,
+  WS_TVG2,
+  WS_TVX2,
   WS_PARTIALS,
   WS_SCALARS,
   WS_FILT,
@@ -217,6 +219,17 @@ struct mexct_ctx {
       b.cap = cap;
     }
     *out = b.p;
+    return MEXCT_OK;
+  }
+
+  int drop(int slot) {
+    Buf& b = ws[slot];
+    if (b.p) {
+      HIPCHK(hipStreamSynchronize(stream));
+      HIPCHK(hipFree(b.p));
+      b.p = nullptr;
+      b.cap = 0;
+    }
     return MEXCT_OK;
   }
 
@@ -1455,11 +1468,26 @@ int mexct_osc_iter(float* mu, int64_t W, int64_t H, float* pre, float* post, int
 // ------------------------------------------------------------------ TV
 namespace {
 int tv_run(mexct_ctx* c, Vol3 x, const float* c_dev, float cc, int steps) {
-  void *gp, *pp, *sp;
-  RC(c->get(WS_TVG, (size_t)x.nx * x.ny * x.nz * 4, &gp));
+  void *gp, *pp, *sp, *g2 = nullptr, *x2 = nullptr;
+  const size_t vb = (size_t)x.nx * x.ny * x.nz * 4;
+  RC(c->get(WS_TVG, vb, &gp));
   RC(c->get(WS_PARTIALS, tv_partials_count(x.nx, x.ny, x.nz) * 8, &pp));
   RC(c->get(WS_SCALARS, 256, &sp));
-  HIPCHK(launch_tvmin(x, (float*)gp, (double*)pp, (float*)sp, c_dev, cc, steps, c->stream));
+  // two volumes more for steps that carry the update along; a volume above
+  // 16 GiB (2^32 voxels), or memory that does not hold them, takes an update pass per step
+  TVWork w;
+  if (steps > 1 && vb <= ((size_t)16 << 30) && c->get(WS_TVG2, vb, &g2) == MEXCT_OK) {
+    if (c->get(WS_TVX2, vb, &x2) == MEXCT_OK) {
+      w.g2 = (float*)g2;
+      w.x2 = (float*)x2;
+    } else {
+      RC(c->drop(WS_TVG2));
+    }
+  }
+  w.g = (float*)gp;
+  w.partials = (double*)pp;
+  w.a_dev = (float*)sp;
+  HIPCHK(launch_tvmin(x, w, c_dev, cc, steps, false, c->stream));
   return MEXCT_OK;
 }
 }  // namespace
@@ -2024,8 +2052,14 @@ int osc_tv_run(mexct_ctx* c, const float* pre, const float* post, int64_t W, int
     if (k > 1) {
       HIPCHK(launch_diff_norm(old_v, mu_v, (double*)pp, sum, st));
       HIPCHK(launch_tv_const(sum, tv, cdev, st));
-      HIPCHK(launch_tvmin(mu_v, (float*)gp, (double*)pp, adev, cdev, 0.f, steps, st));
-      HIPCHK(launch_clean(mu_v, st));
+      // the previous mu and the start volume are not needed any more
+      TVWork w;
+      w.g = (float*)gp;
+      w.g2 = (float*)plain;
+      w.x2 = (float*)mo;
+      w.partials = (double*)pp;
+      w.a_dev = adev;
+      HIPCHK(launch_tvmin(mu_v, w, cdev, 0.f, steps, true, st));
     }
   }
   HIPCHK(launch_unpad3((const float*)mp, mu_out, (int)W, (int)W, (int)H, st));

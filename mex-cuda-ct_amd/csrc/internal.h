@@ -255,11 +255,20 @@ struct Vol3 {
   int nx, ny, nz;
   int64_t sy, sz;
 };
-// `steps` TV gradient steps on x in place.  c is read from c_dev when it is
-// not null, else from `c`.  g ([nx,ny,nz]), partials (tv_partials_count
-// doubles) and a_dev (one float) are workspace.
-hipError_t launch_tvmin(Vol3 x, float* g, double* partials, float* a_dev, const float* c_dev,
-                        float c, int steps, hipStream_t st);
+// Workspace of launch_tvmin: one or two gradients ([nx,ny,nz] each), a second
+// volume of as many floats (with g2), tv_partials_count doubles and a float.
+struct TVWork {
+  float* g;
+  float* g2 = nullptr;  // null: an update pass after every step instead
+  float* x2 = nullptr;
+  double* partials;
+  float* a_dev;
+};
+// `steps` >= 1 TV gradient steps on x in place, the same bits with and without
+// g2.  c is read from c_dev when it is not null, else from `c`.  clean: NaN and
+// +-Inf of the result -> 0 (OSC_TV_recon.m:316-317).
+hipError_t launch_tvmin(Vol3 x, const TVWork& w, const float* c_dev, float c, int steps, bool clean,
+                        hipStream_t st);
 size_t tv_partials_count(int nx, int ny, int nz);
 
 // ---- OSC-TV driver helpers (tv.hip)
@@ -269,8 +278,6 @@ hipError_t launch_diff_norm(Vol3 old_v, Vol3 new_v, double* partials, double* su
                             hipStream_t st);
 // *c_dev = tv * (float)sqrt(*sum)  (OSC_TV_recon.m:314-315)
 hipError_t launch_tv_const(const double* sum, float tv, float* c_dev, hipStream_t st);
-// NaN and +-Inf -> 0 (OSC_TV_recon.m:316-317)
-hipError_t launch_clean(Vol3 x, hipStream_t st);
 
 // ---- FDK prefilter (fdk.hip)
 // The staged sample: x = sino[e], or -log(post[e] / sino[e]) with NaN/Inf
