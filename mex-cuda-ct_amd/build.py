@@ -23,7 +23,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libmexct.so")
-SOURCES = ["pad.hip", "fp.hip", "fpz.hip", "fpc.hip", "bp.hip", "bpc.hip", "g3dbp.hip", "tv.hip", "fdk.hip", "probe.hip",
+SOURCES = ["pad.hip", "fp.hip", "fpz.hip", "fpc.hip", "bp.hip", "bpc.hip", "bpl.hip", "g3dbp.hip", "tv.hip", "fdk.hip", "probe.hip",
            "api.hip", "serve.hip"]
 HEADERS = ["common.h", "internal.h", "ray.h"]
 ARCH = os.environ.get("MEXCT_ARCH", "gfx950")

@@ -668,13 +668,17 @@ size_t op_workspace_bytes(int op, int geom, int st, int64_t W, int64_t H, int64_
     bool zc;
     const int zh = bp_row_halo(W, H, geom, sad, rows, st, &zc);
     size_t vb = (size_t)(W + 4) * (H + 2 * zh - 1) * rows * es;
-    (void)bpc_shape(W, H, geom, sad, st, nullptr, &vb);
+    int lchain = 0;
+    const bool lds = geom == GEOM_CONE && st == MEXCT_F32 &&
+                     bpl_shape(W, H, sad, (int)nitems, nullptr, nullptr, &lchain, &vb);
+    if (!lds) (void)bpc_shape(W, H, geom, sad, st, nullptr, &vb);
     b += slot(vb * n * nitems);
     if (geom == 2 && st == MEXCT_F32) {
       size_t cfv = 0;  // the largest chain of any tuning candidate
       for (int sup : {2, 4, 8})
         for (int zr : {32, 48, 64})
-          cfv = std::max(cfv, bp_chain_floats_per_view((int)W, (int)H, zr, sup));
+          if (!lds || zr == lchain)
+            cfv = std::max(cfv, bp_chain_floats_per_view((int)W, (int)H, zr, sup));
       if (cfv > 0) {
         const size_t cv = std::min<size_t>(n, std::max<size_t>(1, ((size_t)1 << 28) / cfv));
         b += slot(cv * cfv * 4);
@@ -935,6 +939,13 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
   if ((double)W * W * H >= 4294967296.0) return fail(MEXCT_EINVAL, "volume too large");
   // par and fan: by detector columns, on a copy of single rows
   const bool col = bpc_shape(W, H, geom, sad, st, nullptr, &rp_bytes);
+  // cone f32: gathered from LDS, on a copy of single rows with a row halo
+  int lzt = -1, lpv = 0, lchain = 0;
+  const bool lds = geom == GEOM_CONE && st == MEXCT_F32 &&
+                   bpl_shape(W, H, sad, items, &lzt, &lpv, &lchain, &rp_bytes);
+  auto launch = [&](const BPLaunch& l) {
+    return col ? launch_bpc(l, c->stream) : lds ? launch_bpl(l, c->stream) : launch_bp(l, c->stream);
+  };
   DevGuard g(c->device);
   void* pad;
   const size_t sino_stride = rp_bytes * (size_t)std::max<int64_t>(nProj, 1);
@@ -949,10 +960,10 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
       const void* in = in_ptrs ? in_ptrs[i] : (const char*)sino + i * sel * in_es;
       const uint32_t* m = smax ? smax + i : nullptr;
       void* o = (char*)pad + i * sino_stride;
-      HIPCHK(col ? launch_pad2c(in, sino_dtype, o, st, (int)W, (int)H, (int)nProj,
-                                bpc_rows(H, st), c->stream, m)
-                 : launch_pad2(in, sino_dtype, o, st, (int)W, (int)H, (int)nProj, ADDR_CLAMP,
-                               c->stream, m, rows, zh));
+      HIPCHK(col || lds ? launch_pad2c(in, sino_dtype, o, st, (int)W, (int)H, (int)nProj,
+                                       lds ? lpv : bpc_rows(H, st), c->stream, m, lzt)
+                        : launch_pad2(in, sino_dtype, o, st, (int)W, (int)H, (int)nProj, ADDR_CLAMP,
+                                      c->stream, m, rows, zh));
     }
   const float2* sc = nullptr;
   RC(c->sincos_table(angles, (int)nProj, &sc));
@@ -967,7 +978,7 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
   a.H = (int)H;
   a.nviews = (int)nProj;
   a.sad = sad;
-  a.zr = pick_zrange(opts, geom, H);
+  a.zr = lds ? lchain : pick_zrange(opts, geom, H);
   a.rows = rows;
   a.zh = zh;
   a.zclamp = zclamp;
@@ -985,7 +996,7 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
   // candidates: super-tile side 2, 4, 8; the z-range too for FP32 storage
   // unless the caller fixed it
   const bool zr_free =
-      st == MEXCT_F32 && !(opts && (opts->zrange == 32 || opts->zrange == 48 || opts->zrange == 64));
+      st == MEXCT_F32 && !lds && !(opts && (opts->zrange == 32 || opts->zrange == 48 || opts->zrange == 64));
   std::vector<std::pair<int, int>> cand;
   for (int sup : {2, 4, 8}) {
     if (zr_free)
@@ -1019,13 +1030,13 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
   if (tune) {
     int dflt = 0;  // the built-in choice: super-tile 4 at the default z-range
     for (size_t i = 0; i < cand.size(); ++i)
-      if (cand[i].first == 4 && cand[i].second == pick_zrange(opts, geom, H)) dflt = (int)i;
+      if (cand[i].first == 4 && cand[i].second == a.zr) dflt = (int)i;
     const int best = tune_pick(c, (int)cand.size(), dflt, [&](int i) {
       BPLaunch t = a;
       t.super_ = cand[i].first;
       t.zr = cand[i].second;
       t.nviews = (int)std::min<int64_t>(nProj, kTuneViews);
-      HIPCHK(col ? launch_bpc(t, c->stream) : launch_bp(t, c->stream));
+      HIPCHK(launch(t));
       return MEXCT_OK;
     }, &tv.ms);
     if (best < 0) return best;
@@ -1035,7 +1046,7 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
     a.super_ = tv.a;
     if (zr_free) a.zr = tv.b;
   }
-  HIPCHK(col ? launch_bpc(a, c->stream) : launch_bp(a, c->stream));
+  HIPCHK(launch(a));
   return MEXCT_OK;
 }
 }  // namespace

@@ -461,6 +461,29 @@ size_t bp_chain_floats_per_view(int W, int H, int zr, int super_) {
   return nz > 1 ? (size_t)tpad * tpad * 64u * (nz - 1) : 0;
 }
 
+hipError_t launch_bp_chain(const float2* sc, int nviews, int W, int H, float sad, int zr, int super_,
+                           float* chain, hipStream_t st) {
+  BPKArgs k{};
+  k.sc = sc;
+  k.W = W;
+  k.nviews = nviews;
+  k.v0 = float(H - 1) / 2;
+  k.SR = sad;
+  k.super_ = super_ > 0 ? (uint32_t)super_ : kSuper;
+  k.tiles_x = (uint32_t)((W + 7) / 8);
+  k.nz = (uint32_t)((H + zr - 1) / zr);
+  const uint32_t tpad = (k.tiles_x + k.super_ - 1) / k.super_ * k.super_;
+  k.ncols = tpad * tpad * 64u;
+  const unsigned g = (unsigned)std::min<size_t>(((size_t)k.ncols * nviews + 255) / 256, 65536);
+  if (zr == 64)
+    bp_chain_kernel<64><<<g, 256, 0, st>>>(k, chain);
+  else if (zr == 48)
+    bp_chain_kernel<48><<<g, 256, 0, st>>>(k, chain);
+  else
+    bp_chain_kernel<32><<<g, 256, 0, st>>>(k, chain);
+  return hipGetLastError();
+}
+
 // Views go in chunks whose row-paired slices stay below 2 GiB (32-bit
 // buffer offsets); each chunk continues the register sums the previous one
 // stored, so the per-voxel order and the float sums are unchanged.
@@ -509,14 +532,8 @@ hipError_t launch_bp(const BPLaunch& a, hipStream_t st) {
     k.accumulate = v0 > 0;
     k.chain = nullptr;
     if (use_chain && cn > 0) {
-      const size_t total = (size_t)k.ncols * cn;
-      const unsigned cg = (unsigned)std::min<size_t>((total + 255) / 256, 65536);
-      if (zr == 64)
-        bp_chain_kernel<64><<<cg, 256, 0, st>>>(k, a.chain);
-      else if (zr == 48)
-        bp_chain_kernel<48><<<cg, 256, 0, st>>>(k, a.chain);
-      else
-        bp_chain_kernel<32><<<cg, 256, 0, st>>>(k, a.chain);
+      const hipError_t e = launch_bp_chain(k.sc, cn, a.W, a.H, a.sad, zr, (int)k.super_, a.chain, st);
+      if (e != hipSuccess) return e;
       k.chain = a.chain;
     }
     if (a.st_dt == 0)

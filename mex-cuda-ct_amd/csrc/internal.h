@@ -49,9 +49,11 @@ hipError_t launch_pad2(const void* in, int in_dt, void* out, int st_dt, int w, i
                        int rows = 2, int zh = 2);
 // Sinogram copy for the column backprojector (bpc.hip): in [w,h,n] ->
 // out[(view*(w+4) + u+2)*pv + v], pv >= h rows per detector column (bpc_rows).
-// A value is NaN where it or the one at v+1 is not finite.
+// zt < 0: rows 0 .. h-1, then zeros; a value is NaN where it or the one at v+1
+// is not finite.  zt >= 0 (bpl.hip): row v holds detector row v - zt, edge copies
+// outside.
 hipError_t launch_pad2c(const void* in, int in_dt, void* out, int st_dt, int w, int h, int n, int pv,
-                        hipStream_t st, const uint32_t* scale_max = nullptr);
+                        hipStream_t st, const uint32_t* scale_max = nullptr, int zt = -1);
 // scale_max (pad3z, pad3q, pad2): when non-null, the bits of max|in|; the
 // copy holds in * 2^-pow2_exp(scale_max) (see common.h).
 // 3D interior copy between a padded f32 volume and a plain one.
@@ -173,6 +175,18 @@ struct BPLaunch {
   int zh = 2;
   bool zclamp = true;
 };
+// Row coordinates of the cone's running sum at every zr-th slice (32, 48 or 64),
+// chain[(view*(ceil(H/zr) - 1) + r - 1)*ncols + col] for slice r*zr
+// (bp_chain_floats_per_view floats per view).
+hipError_t launch_bp_chain(const float2* sc, int nviews, int W, int H, float sad, int zr, int super_,
+                           float* chain, hipStream_t st);
+// Cone f32 with the detector in LDS (bpl.hip): a launch_pad2c copy of pv rows, zt
+// of them edge copies before row 0, and a chain every chain_slices; false for
+// shapes it does not take.  The same arguments and bits as launch_bp (zr:
+// chain_slices; rows, zh, zclamp unused).
+bool bpl_shape(int64_t W, int64_t H, float sad, int items, int* zt, int* pv, int* chain_slices,
+               size_t* view_bytes);
+hipError_t launch_bpl(const BPLaunch& a, hipStream_t st);
 // floats of BP chain scratch per view (cone f32, z-range zr, super-tile side)
 size_t bp_chain_floats_per_view(int W, int H, int zr, int super_);
 hipError_t launch_bp(const BPLaunch& a, hipStream_t st);

@@ -82,22 +82,23 @@ __global__ __launch_bounds__(256) void pad2_kernel(const void* __restrict__ in, 
   }
 }
 
-// Sinogram copy for the column backprojector (see launch_pad2c): row-fastest,
-// out[(view*(w+4) + u+2)*pv + v], edge copies at u = -2, -1, w, w+1, zeros at
-// v >= h.  A block covers 32 u x 32 v of one view through LDS, read along u
-// and written along v.  A value is stored as NaN where it or the one at v + 1
-// is not finite in the storage type (what the weight-0 row lerp makes of them).
+// Sinogram copy for the column and LDS backprojectors (see launch_pad2c):
+// row-fastest, out[(view*(w+4) + u+2)*pv + v], edge copies at u = -2, -1, w, w+1.
+// A block covers 32 u x 32 v of one view through LDS, read along u and written
+// along v.  zt < 0: zeros at v >= h, and a value is stored as NaN where it or
+// the one at v + 1 is not finite in the storage type (what the weight-0 row lerp
+// makes of them).  zt >= 0: row v is detector row v - zt, edge copies outside.
 template <typename S>
 __global__ __launch_bounds__(256) void pad2c_kernel(const void* __restrict__ in, int in_dt,
                                                     S* __restrict__ out, int w, int h, int pv,
-                                                    const uint32_t* scale_max) {
+                                                    const uint32_t* scale_max, int zt) {
   __shared__ float tile[33][33];
   const int sexp = pow2_exp(scale_max);
   const int v0 = blockIdx.x * 32, pu0 = blockIdx.y * 32;
   const size_t vbase = (size_t)w * h * blockIdx.z;
   for (int e = threadIdx.x; e < 33 * 32; e += 256) {
     const int lv = e >> 5, lu = e & 31;
-    const int i = clampi(pu0 + lu - HALO, 0, w - 1), j = clampi(v0 + lv, 0, h - 1);
+    const int i = clampi(pu0 + lu - HALO, 0, w - 1), j = clampi(v0 + lv - max(zt, 0), 0, h - 1);
     const S t = Store<S>::from(ldexpf(load_any(in, in_dt, (size_t)i + (size_t)w * j + vbase), -sexp));
     tile[lv][lu] = Store<S>::ld(&t);
   }
@@ -107,8 +108,10 @@ __global__ __launch_bounds__(256) void pad2c_kernel(const void* __restrict__ in,
     const int lu = tu + 8 * p, pu = pu0 + lu, v = v0 + tv;
     if (pu >= w + 2 * HALO || v >= pv) continue;
     const float x = tile[tv][lu], n = tile[tv + 1][lu];
-    const float y = v >= h ? 0.f
-                    : __builtin_isfinite(x) && __builtin_isfinite(n) ? x : __builtin_nanf("");
+    const float y = zt >= 0  ? x
+                    : v >= h ? 0.f
+                    : __builtin_isfinite(x) && __builtin_isfinite(n) ? x
+                                                                    : __builtin_nanf("");
     out[((size_t)blockIdx.z * (w + 2 * HALO) + pu) * pv + v] = Store<S>::from(y);
   }
 }
@@ -409,7 +412,7 @@ hipError_t launch_pad2(const void* in, int in_dt, void* out, int st_dt, int w, i
 }
 
 hipError_t launch_pad2c(const void* in, int in_dt, void* out, int st_dt, int w, int h, int n, int pv,
-                        hipStream_t st, const uint32_t* scale_max) {
+                        hipStream_t st, const uint32_t* scale_max, int zt) {
   const size_t es = st_dt == 0 ? 4 : 2, ies = in_dt == 0 ? 4 : 2;
   for (int v = 0; v < n; v += 65535) {  // the grid's z extent
     const dim3 g((unsigned)((pv + 31) / 32), (unsigned)((w + 2 * HALO + 31) / 32),
@@ -417,11 +420,11 @@ hipError_t launch_pad2c(const void* in, int in_dt, void* out, int st_dt, int w, 
     const void* i = (const char*)in + (size_t)v * w * h * ies;
     void* o = (char*)out + (size_t)v * (w + 2 * HALO) * pv * es;
     if (st_dt == 0)
-      pad2c_kernel<float><<<g, 256, 0, st>>>(i, in_dt, (float*)o, w, h, pv, scale_max);
+      pad2c_kernel<float><<<g, 256, 0, st>>>(i, in_dt, (float*)o, w, h, pv, scale_max, zt);
     else if (st_dt == 1)
-      pad2c_kernel<_Float16><<<g, 256, 0, st>>>(i, in_dt, (_Float16*)o, w, h, pv, scale_max);
+      pad2c_kernel<_Float16><<<g, 256, 0, st>>>(i, in_dt, (_Float16*)o, w, h, pv, scale_max, zt);
     else
-      pad2c_kernel<bf16_t><<<g, 256, 0, st>>>(i, in_dt, (bf16_t*)o, w, h, pv, scale_max);
+      pad2c_kernel<bf16_t><<<g, 256, 0, st>>>(i, in_dt, (bf16_t*)o, w, h, pv, scale_max, zt);
   }
   return hipGetLastError();
 }
