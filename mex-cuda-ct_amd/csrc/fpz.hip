@@ -11,7 +11,8 @@
 // about one line per lane.  A 256-thread workgroup holds 4 adjacent
 // columns.  Loads are 32-bit buffer offsets.
 //
-// Three z-fastest layouts, each haloed by 2 on every side:
+// Three z-fastest layouts, each haloed by 2 on every side (DUAL and QUAD rows
+// fp_zrow elements apart):
 //   PLAIN: V(x,y,z); per sample four (z, z+1) pair loads at the (j+1),
 //     (i+1), (i+1,j+1) strides in scalar offsets.
 //   DUAL (f32): element (x,y,z) = {V(x,y,z), V(x+1,y,z)}; the two elements
@@ -630,7 +631,7 @@ static FPZArgs make_zargs(const void* vol, int st_dt, int layout_, const float2*
   // corner pair or quad, whose base runs over [-2, N] (N+3)
   const int PX = layout == LAYOUT_PLAIN ? NX + 2 * HALO : NX + 2 * HALO - 1;
   k.PY = layout == LAYOUT_QUAD ? NX + 2 * HALO - 1 : NX + 2 * HALO;
-  k.PZ = NZ + 2 * HALO;
+  k.PZ = layout == LAYOUT_PLAIN ? NZ + 2 * HALO : (int)fp_zrow(NX, NZ);
   k.PYPZ = k.PY * k.PZ;
   const uint32_t es = (st_dt == 0 ? 4u : 2u) *
                       (layout == LAYOUT_QUAD ? 4u : layout == LAYOUT_DUAL ? 2u : 1u);

@@ -20,14 +20,31 @@ hipError_t launch_pad3(const void* in, int in_dt, void* out, int st_dt, int nx, 
 hipError_t launch_pad3z(const void* in, int in_dt, int64_t in_sy, int64_t in_sz, void* out,
                         int st_dt, int nx, int ny, int nz, int mode, hipStream_t st,
                         const uint32_t* scale_max = nullptr);
+// Elements (of 8 bytes) from one z row of the dual and quad copies of an
+// n x n x nz volume to the next: the nz + 4 of the row, or, where that is within
+// 64 bytes of a multiple of 4096 bytes, 128 bytes more than the multiple (unless
+// the copy would lose its 32-bit forms).  The projectors gather a few lines of
+// each of many rows at a time, which from rows about 4096 bytes apart meet in
+// few sets of the L2s: cone f16, 400 views of 512 x H: H = 500 (4032 bytes) 31.2 ms,
+// 504 54.9, 508 36.2, 512 57.4, 516 32.7, 520 (4192 bytes) 31.1; with the longer
+// rows 30.8, 30.9, 31.2 and 31.3 ms at 504 to 516.  Other rows stay as tight as
+// they are: whole odd numbers of lines ran the general-3D projection 9% slower.
+inline int64_t fp_zrow(int64_t n, int64_t nz) {
+  const int64_t tight = nz + 4, m = (tight + 8) / 512 * 512;  // the multiple at or 64 bytes above
+  const int64_t p = m + 16;
+  if (m == 0 || tight > m + 8 || (n + 4) * p >= ((int64_t)1 << 23) ||
+      (n + 3) * (n + 4) * p >= ((int64_t)1 << 29))
+    return tight;
+  return p;
+}
 // z-fastest x-pair ("dual") copy: element (x,y,z), x in [-2,n], y, z in
-// [-2, n+1] / [-2, nz+1], at ((x+2)*(ny+4) + y+2)*(nz+4) + z+2 holds
+// [-2, n+1] / [-2, nz+1], at ((x+2)*(ny+4) + y+2)*fp_zrow + z+2 holds
 // {V(x,y,z), V(x+1,y,z)} of the haloed volume V.
 hipError_t launch_pad3d(const void* in, int in_dt, int64_t in_sy, int64_t in_sz, void* out,
                         int st_dt, int nx, int ny, int nz, int mode, hipStream_t st,
                         const uint32_t* scale_max = nullptr);
 // z-fastest corner-quad copy: element (x,y,z), x,y in [-2,n], z in [-2,nz+1], at
-// ((x+2)*(ny+3) + y+2)*(nz+4) + z+2 holds {V(x,y,z), V(x,y+1,z), V(x+1,y,z),
+// ((x+2)*(ny+3) + y+2)*fp_zrow + z+2 holds {V(x,y,z), V(x,y+1,z), V(x+1,y,z),
 // V(x+1,y+1,z)} of the haloed volume V (same input addressing as launch_pad3z);
 // f16 holds the differences {V, Dy, Dx, Dxy} of those four instead (pad.hip).
 hipError_t launch_pad3q(const void* in, int in_dt, int64_t in_sy, int64_t in_sz, void* out,

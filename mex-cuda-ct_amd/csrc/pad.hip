@@ -179,7 +179,7 @@ template <typename S>
 __global__ __launch_bounds__(256) void pad3d_kernel(const void* __restrict__ in, int in_dt,
                                                     int64_t in_sy, int64_t in_sz,
                                                     S* __restrict__ out, int nx, int ny, int nz,
-                                                    int mode, const uint32_t* scale_max) {
+                                                    int pz, int mode, const uint32_t* scale_max) {
   __shared__ float tile[32][33];
   const int sexp = pow2_exp(scale_max);
   const int DX = nx + 2 * HALO - 1, DY = ny + 2 * HALO, DZ = nz + 2 * HALO;
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void pad3d_kernel(const void* __restrict__ in,
     const int lx = ty + 8 * p;
     const int dx = dx0 + lx, dz = dz0 + tz;
     if (dx < DX && dz < DZ) {
-      const size_t e = ((size_t)dx * DY + dy) * DZ + dz;
+      const size_t e = ((size_t)dx * DY + dy) * pz + dz;
       store_pair<S>(out + 2 * e, tile[tz][lx], tile[tz][lx + 1]);
     }
   }
@@ -254,7 +254,7 @@ template <typename S>
 __global__ __launch_bounds__(256) void pad3q_kernel(const void* __restrict__ in, int in_dt,
                                                     int64_t in_sy, int64_t in_sz,
                                                     S* __restrict__ out, int nx, int ny, int nz,
-                                                    int mode, const uint32_t* scale_max) {
+                                                    int pz, int mode, const uint32_t* scale_max) {
   __shared__ float tile[2][32][33];
   const int sexp = pow2_exp(scale_max);
   const int QX = nx + 2 * HALO - 1, QY = ny + 2 * HALO - 1, QZ = nz + 2 * HALO;
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(256) void pad3q_kernel(const void* __restrict__ in,
     const int lx = ty + 8 * p;
     const int qx = qx0 + lx, qz = qz0 + tz;
     if (qx < QX && qz < QZ)
-      Quad<S>::put(out, ((size_t)qx * QY + qy) * QZ + qz, tile[0][tz][lx], tile[1][tz][lx],
+      Quad<S>::put(out, ((size_t)qx * QY + qy) * pz + qz, tile[0][tz][lx], tile[1][tz][lx],
                    tile[0][tz][lx + 1], tile[1][tz][lx + 1]);
   }
 }
@@ -434,14 +434,15 @@ hipError_t launch_pad3d(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
                         const uint32_t* scale_max) {
   const dim3 g((unsigned)((nz + 2 * HALO + 31) / 32), (unsigned)((nx + 2 * HALO - 1 + 31) / 32),
                (unsigned)(ny + 2 * HALO));
+  const int pz = (int)fp_zrow(nx, nz);
   if (st_dt == 0)
-    pad3d_kernel<float><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (float*)out, nx, ny, nz, mode,
-                                           scale_max);
+    pad3d_kernel<float><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (float*)out, nx, ny, nz, pz,
+                                           mode, scale_max);
   else if (st_dt == 1)
     pad3d_kernel<_Float16><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (_Float16*)out, nx, ny, nz,
-                                              mode, scale_max);
+                                              pz, mode, scale_max);
   else
-    pad3d_kernel<bf16_t><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (bf16_t*)out, nx, ny, nz,
+    pad3d_kernel<bf16_t><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (bf16_t*)out, nx, ny, nz, pz,
                                             mode, scale_max);
   return hipGetLastError();
 }
@@ -451,13 +452,15 @@ hipError_t launch_pad3q(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
                         const uint32_t* scale_max) {
   const dim3 g((unsigned)((nz + 2 * HALO + 31) / 32), (unsigned)((nx + 2 * HALO - 1 + 31) / 32),
                (unsigned)(ny + 2 * HALO - 1));
+  const int pz = (int)fp_zrow(nx, nz);
   if (st_dt == 0)
-    pad3q_kernel<float><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (float*)out, nx, ny, nz, mode, scale_max);
+    pad3q_kernel<float><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (float*)out, nx, ny, nz, pz,
+                                           mode, scale_max);
   else if (st_dt == 1)
     pad3q_kernel<_Float16><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (_Float16*)out, nx, ny, nz,
-                                              mode, scale_max);
+                                              pz, mode, scale_max);
   else
-    pad3q_kernel<bf16_t><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (bf16_t*)out, nx, ny, nz,
+    pad3q_kernel<bf16_t><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (bf16_t*)out, nx, ny, nz, pz,
                                             mode, scale_max);
   return hipGetLastError();
 }
