@@ -376,7 +376,7 @@ int fp_layout(int geom, int64_t W, int64_t H, int st, size_t* bytes) {
   const bool force64 = force && !strcmp(force, "wide64");
   const int want = st == MEXCT_F32 ? LAYOUT_DUAL : LAYOUT_QUAD;
   const size_t elems =
-      (size_t)(W + 3) * (want == LAYOUT_DUAL ? W + 4 : W + 3) * (size_t)fp_zrow(W, H);
+      (size_t)(W + 3) * (want == LAYOUT_DUAL ? W + 4 : W + 3) * (size_t)fp_zrow(W, H, want == LAYOUT_DUAL);
   *bytes = elems * (want == LAYOUT_DUAL ? 2 : 4) * es;
   if (*bytes < ((size_t)1 << 32) && !force64) return want;
   if (elems < ((size_t)1 << 32)) return want == LAYOUT_DUAL ? LAYOUT_DUAL64 : LAYOUT_QUAD64;

@@ -631,7 +631,7 @@ static FPZArgs make_zargs(const void* vol, int st_dt, int layout_, const float2*
   // corner pair or quad, whose base runs over [-2, N] (N+3)
   const int PX = layout == LAYOUT_PLAIN ? NX + 2 * HALO : NX + 2 * HALO - 1;
   k.PY = layout == LAYOUT_QUAD ? NX + 2 * HALO - 1 : NX + 2 * HALO;
-  k.PZ = layout == LAYOUT_PLAIN ? NZ + 2 * HALO : (int)fp_zrow(NX, NZ);
+  k.PZ = layout == LAYOUT_PLAIN ? NZ + 2 * HALO : (int)fp_zrow(NX, NZ, layout == LAYOUT_DUAL);
   k.PYPZ = k.PY * k.PZ;
   const uint32_t es = (st_dt == 0 ? 4u : 2u) *
                       (layout == LAYOUT_QUAD ? 4u : layout == LAYOUT_DUAL ? 2u : 1u);

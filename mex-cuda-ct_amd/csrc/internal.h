@@ -29,13 +29,15 @@ hipError_t launch_pad3z(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
 // 504 54.9, 508 36.2, 512 57.4, 516 32.7, 520 (4192 bytes) 31.1; with the longer
 // rows 30.8, 30.9, 31.2 and 31.3 ms at 504 to 516.  Other rows stay as tight as
 // they are: whole odd numbers of lines ran the general-3D projection 9% slower.
-inline int64_t fp_zrow(int64_t n, int64_t nz) {
+// The dual copy, of which a sample loads two rows, takes rows of 48 or 80 bytes
+// past a multiple of 128, the best of 12 rows tried at six sizes: cone 384^3 x 512
+// views 25.6 -> 24.5 ms, 256^3 x 360 5.27 -> 5.11, general-3D 320^3 x 360 22.2 ->
+// 21.4, 250^2 x 187 x 240 8.70 -> 8.04; the quads show no such order.
+inline int64_t fp_zrow(int64_t n, int64_t nz, bool dual) {
   const int64_t tight = nz + 4, m = (tight + 8) / 512 * 512;  // the multiple at or 64 bytes above
-  const int64_t p = m + 16;
-  if (m == 0 || tight > m + 8 || (n + 4) * p >= ((int64_t)1 << 23) ||
-      (n + 3) * (n + 4) * p >= ((int64_t)1 << 29))
-    return tight;
-  return p;
+  int64_t p = m == 0 || tight > m + 8 ? tight : m + 16;
+  while (dual && p % 16 != 6 && p % 16 != 10) ++p;
+  return (n + 4) * p >= ((int64_t)1 << 23) || (n + 3) * (n + 4) * p >= ((int64_t)1 << 29) ? tight : p;
 }
 // z-fastest x-pair ("dual") copy: element (x,y,z), x in [-2,n], y, z in
 // [-2, n+1] / [-2, nz+1], at ((x+2)*(ny+4) + y+2)*fp_zrow + z+2 holds

@@ -434,7 +434,7 @@ hipError_t launch_pad3d(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
                         const uint32_t* scale_max) {
   const dim3 g((unsigned)((nz + 2 * HALO + 31) / 32), (unsigned)((nx + 2 * HALO - 1 + 31) / 32),
                (unsigned)(ny + 2 * HALO));
-  const int pz = (int)fp_zrow(nx, nz);
+  const int pz = (int)fp_zrow(nx, nz, true);
   if (st_dt == 0)
     pad3d_kernel<float><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (float*)out, nx, ny, nz, pz,
                                            mode, scale_max);
@@ -452,7 +452,7 @@ hipError_t launch_pad3q(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
                         const uint32_t* scale_max) {
   const dim3 g((unsigned)((nz + 2 * HALO + 31) / 32), (unsigned)((nx + 2 * HALO - 1 + 31) / 32),
                (unsigned)(ny + 2 * HALO - 1));
-  const int pz = (int)fp_zrow(nx, nz);
+  const int pz = (int)fp_zrow(nx, nz, false);
   if (st_dt == 0)
     pad3q_kernel<float><<<g, 256, 0, st>>>(in, in_dt, in_sy, in_sz, (float*)out, nx, ny, nz, pz,
                                            mode, scale_max);
