@@ -7,7 +7,8 @@
 // linear convolution y[u] = sum_u' x[u'] h[(u - u') mod order] with the
 // filter's circular impulse response h, so each row is filtered here by a
 // direct FP64 convolution against the 2W-1 taps g[d] = h[d mod order],
-// d in [-(W-1), W-1], staged once per workgroup in LDS.  The cosine weight
+// d in [-(W-1), W-1], staged once per workgroup in LDS: on the matrix cores for
+// rows of up to 768 samples, an output per thread above.  The cosine weight
 // (:51-58, single * single) is applied while the row is staged, and the
 // angle-step scale (:80-84) in single precision on the way out.
 //
@@ -21,18 +22,27 @@ namespace mexct {
 
 constexpr int FDK_THREADS = 256;
 
-// Sample u of detector row v of view `view`, weighted as the filter expects.
-__device__ __forceinline__ float stage_sample(const FilterIn& in, size_t base, int view, int v,
-                                              int u, int W) {
-  float x;
+// Sample u of detector row v of view `view` as loaded, and weighted as the
+// filter expects.
+struct RawSample {
+  float x, post, wgt, pw;
+};
+__device__ __forceinline__ RawSample load_sample(const FilterIn& in, size_t base, int view, int v,
+                                                 int u, int W) {
+  RawSample r{in.sino[base + u], 0.f, 0.f, 0.f};
+  if (in.post) r.post = in.post[base + u];
+  if (in.wgt) r.wgt = in.wgt[(size_t)v * W + u];
+  if (in.pw) r.pw = in.pw[(size_t)view * W + u];
+  return r;
+}
+__device__ __forceinline__ float weigh_sample(const FilterIn& in, const RawSample& r) {
+  float x = r.x;
   if (in.post) {
-    x = -logf(in.post[base + u] / in.sino[base + u]);
+    x = -logf(r.post / r.x);
     if (!__builtin_isfinite(x)) x = 0.f;
-  } else {
-    x = in.sino[base + u];
   }
-  if (in.wgt) x = x * in.wgt[(size_t)v * W + u];
-  if (in.pw) x = x * in.pw[(size_t)view * W + u];
+  if (in.wgt) x = x * r.wgt;
+  if (in.pw) x = x * r.pw;
   return x;
 }
 
@@ -48,7 +58,7 @@ __global__ __launch_bounds__(FDK_THREADS) void prefilter_kernel(
     const size_t base = (size_t)view * W * H + (size_t)v * W;
     __syncthreads();
     for (int u = threadIdx.x; u < W; u += FDK_THREADS)
-      xs[u] = (double)stage_sample(in, base, view, v, u, W);
+      xs[u] = (double)weigh_sample(in, load_sample(in, base, view, v, u, W));
     __syncthreads();
     const float d = dA[view];
     for (int u = threadIdx.x; u < W; u += FDK_THREADS) {
@@ -61,71 +71,103 @@ __global__ __launch_bounds__(FDK_THREADS) void prefilter_kernel(
   }
 }
 
-// Register-blocked form for W <= 64 R: a wave filters one row, each lane R
-// consecutive outputs.  For a block of R input samples the lane needs the
-// 2R-1 taps g[b-R+1 .. b+R-1] (b = u0 - U0 + W - 1), which it loads once
-// from LDS and reuses for R^2 FMAs.  Every output still sums its products in
-// input order from u' = 0, the same FP64 sum as prefilter_kernel.  Rows are
-// zero-padded to a multiple of R (the extra products add +0) and the taps
-// by zeros on both sides, so no index leaves the LDS arrays.
-template <int R>
-__global__ __launch_bounds__(FDK_THREADS) void prefilter_reg_kernel(
+// Rows of up to 768 samples on the matrix cores: y = x G with the Toeplitz
+// matrix G[u'][u] = g[u - u'], in v_mfma_f64_16x16x4 (16 rows, 4 inputs, 16
+// outputs; every product and sum in FP64).  A workgroup filters 16 MR rows, each
+// of its four waves NT tiles of 16 outputs (wave w the tiles w, w + 4, ...); the
+// rows lie in LDS as floats, an odd number apart, the taps as doubles, zero
+// beyond the row's ends, so a fragment of G is 16 x 4 taps read where its
+// diagonal lies.  Inputs past the row are zero (their products add nothing to a
+// real output), outputs past it are dropped.
+// Bound by the FP64 matrix cores (64 clocks a product per SIMD): busy 67% of the
+// time at 301 samples, 75% at 512, the rest staging.  With the log, against
+// direct FP64 convolutions of R outputs per lane, whose taps came through LDS:
+// 301 x 211 x 250 views 559 -> 248 us; the whole FBP 256^3 x 360 views 5.18 -> 2.73 ms
+// (of which the filter 1.2 -> 0.24), 512^2 x 400 x 400 33.0 -> 23.6 ms, 700^2 x 100 x 200
+// 7.85 -> 7.47 ms.  (256, 2) keeps the sums in VGPRs: with AGPRs the compiler copied all
+// of them each trip, 403 us.  Staging four samples at a time against one: 26% of the
+// kernel at 301.
+template <int MR, int NT>
+__global__ __launch_bounds__(FDK_THREADS, 2) void prefilter_mfma_kernel(
     FilterIn in, float* __restrict__ out, const double* __restrict__ g,
     const float* __restrict__ dA, int W, int H, int nrows) {
+  typedef double d4v __attribute__((ext_vector_type(4)));
   extern __shared__ double lds[];
-  const int Wp = (W + R - 1) / R * R;
-  const int GL = R + 64 * R + W;  // padded tap array: gs[i] = g[i - R]
-  double* gs = lds;
-  double* xs = lds + GL + (threadIdx.x >> 6) * Wp;
+  const int Kp = (W + 3) & ~3, XS = Kp | 1, GL = 64 * NT + Kp;
+  double* const gs = lds;  // gs[Kp - 1 + d] = tap d
+  float* const xs = (float*)(lds + GL);
+  const int row0 = (int)blockIdx.x * (16 * MR);
   for (int i = threadIdx.x; i < GL; i += FDK_THREADS) {
-    const int k = i - R;
-    gs[i] = (k >= 0 && k < 2 * W - 1) ? g[k] : 0.0;
+    const int k = i - Kp + W;
+    gs[i] = k >= 0 && k < 2 * W - 1 ? g[k] : 0.0;
   }
-  const int lane = threadIdx.x & 63;
-  const int u0 = lane * R;
-  for (int row0 = blockIdx.x * 4; row0 < nrows; row0 += gridDim.x * 4) {
-    const int row = row0 + (int)(threadIdx.x >> 6);
-    __syncthreads();
-    if (row < nrows) {
-      const int view = row / H, v = row - view * H;
-      const size_t base = (size_t)view * W * H + (size_t)v * W;
-      for (int u = lane; u < Wp; u += 64)
-        xs[u] = u < W ? (double)stage_sample(in, base, view, v, u, W) : 0.0;
-    }
-    __syncthreads();
-    if (row >= nrows) continue;
-    double acc[R];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int r = wave; r < 16 * MR; r += 4) {
+    const int row = min(row0 + r, nrows - 1);
+    const int view = row / H, v = row - view * H;
+    for (int u0 = lane; u0 < Kp; u0 += 256) {  // four loads of each kind in flight
+      RawSample raw[4];
 #pragma unroll
-    for (int k = 0; k < R; ++k) acc[k] = 0.0;
-    for (int U0 = 0; U0 < Wp; U0 += R) {
-      const double* t0 = gs + R + (u0 - U0 + W - 1) - (R - 1);  // t[i] = g[b - R + 1 + i]
-      double t[2 * R - 1];
+      for (int q = 0; q < 4; ++q)
+        raw[q] = load_sample(in, (size_t)row * W, view, v, min(u0 + 64 * q, W - 1), W);
 #pragma unroll
-      for (int i = 0; i < 2 * R - 1; ++i) t[i] = t0[i];
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        const double x = xs[U0 + j];
-#pragma unroll
-        for (int k = 0; k < R; ++k) acc[k] = __builtin_fma(x, t[k - j + R - 1], acc[k]);
+      for (int q = 0; q < 4; ++q) {
+        const int u = u0 + 64 * q;
+        if (u < Kp) xs[r * XS + u] = u < W ? weigh_sample(in, raw[q]) : 0.f;
       }
     }
-    const int view = row / H, v = row - view * H;
-    const size_t base = (size_t)view * W * H + (size_t)v * W;
-    const float d = dA[view];
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-      if (u0 + k < W) out[base + u0 + k] = ((float)acc[k] * d) / 2.0f;
-    }
   }
+  __syncthreads();
+  d4v acc[MR][NT];
+#pragma unroll
+  for (int m = 0; m < MR; ++m)
+#pragma unroll
+    for (int c = 0; c < NT; ++c) acc[m][c] = d4v{0.0, 0.0, 0.0, 0.0};
+  const int l16 = lane & 15, k4 = lane >> 4;
+  const float* xp = xs + l16 * XS + k4;
+  const double* gp = gs + Kp - 1 + 16 * wave + l16 - k4;
+#pragma unroll 2
+  for (int k0 = 0; k0 < Kp; k0 += 4) {
+    double x[MR], t[NT];
+#pragma unroll
+    for (int m = 0; m < MR; ++m) x[m] = (double)xp[16 * m * XS + k0];
+#pragma unroll
+    for (int c = 0; c < NT; ++c) t[c] = gp[64 * c - k0];
+#pragma unroll
+    for (int c = 0; c < NT; ++c)
+#pragma unroll
+      for (int m = 0; m < MR; ++m)
+        acc[m][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[m], t[c], acc[m][c], 0, 0, 0);
+  }
+  // element q of a lane: row 4 q + lane / 16 of the tile, output lane % 16
+#pragma unroll
+  for (int m = 0; m < MR; ++m)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = row0 + 16 * m + 4 * q + k4;
+      if (row >= nrows) continue;
+      const float d = dA[row / H];
+      float* const o = out + (size_t)row * W;
+#pragma unroll
+      for (int c = 0; c < NT; ++c) {
+        const int u = 64 * c + 16 * wave + l16;
+        if (u < W) o[u] = ((float)acc[m][c][q] * d) / 2.0f;
+      }
+    }
 }
 
-template <int R>
-static hipError_t launch_reg(const FilterIn& in, float* out, const double* g, const float* dA,
-                             int W, int H, int nrows, hipStream_t st) {
-  const int Wp = (W + R - 1) / R * R;
-  const size_t lds = sizeof(double) * (size_t)(R + 64 * R + W + 4 * Wp);
-  const int blocks = std::min((nrows + 3) / 4, 16384);
-  prefilter_reg_kernel<R><<<blocks, FDK_THREADS, lds, st>>>(in, out, g, dA, W, H, nrows);
+template <int NT>
+static hipError_t launch_mfma(const FilterIn& in, float* out, const double* g, const float* dA,
+                              int W, int H, int nrows, hipStream_t st) {
+  const int Kp = (W + 3) & ~3;
+  const size_t taps = sizeof(double) * (size_t)(64 * NT + Kp);
+  // 32 rows per workgroup where that still gives two to every CU
+  if (nrows >= 32 * 512)
+    prefilter_mfma_kernel<2, NT><<<(nrows + 31) / 32, FDK_THREADS, taps + sizeof(float) * 32 * (size_t)(Kp | 1), st>>>(
+        in, out, g, dA, W, H, nrows);
+  else
+    prefilter_mfma_kernel<1, NT><<<(nrows + 15) / 16, FDK_THREADS, taps + sizeof(float) * 16 * (size_t)(Kp | 1), st>>>(
+        in, out, g, dA, W, H, nrows);
   return hipGetLastError();
 }
 
@@ -133,11 +175,20 @@ hipError_t launch_prefilter(const FilterIn& in, float* out, const double* g, con
                             int W, int H, int nviews, hipStream_t st) {
   const int nrows = H * nviews;
   if (nrows == 0) return hipSuccess;
-  if (W <= 64 * 2) return launch_reg<2>(in, out, g, dA, W, H, nrows, st);
-  if (W <= 64 * 4) return launch_reg<4>(in, out, g, dA, W, H, nrows, st);
-  if (W <= 64 * 6) return launch_reg<6>(in, out, g, dA, W, H, nrows, st);
-  if (W <= 64 * 8) return launch_reg<8>(in, out, g, dA, W, H, nrows, st);
-  if (W <= 64 * 12) return launch_reg<12>(in, out, g, dA, W, H, nrows, st);
+  switch ((W + 63) / 64) {
+    case 1: return launch_mfma<1>(in, out, g, dA, W, H, nrows, st);
+    case 2: return launch_mfma<2>(in, out, g, dA, W, H, nrows, st);
+    case 3: return launch_mfma<3>(in, out, g, dA, W, H, nrows, st);
+    case 4: return launch_mfma<4>(in, out, g, dA, W, H, nrows, st);
+    case 5: return launch_mfma<5>(in, out, g, dA, W, H, nrows, st);
+    case 6: return launch_mfma<6>(in, out, g, dA, W, H, nrows, st);
+    case 7: return launch_mfma<7>(in, out, g, dA, W, H, nrows, st);
+    case 8: return launch_mfma<8>(in, out, g, dA, W, H, nrows, st);
+    case 9:
+    case 10: return launch_mfma<10>(in, out, g, dA, W, H, nrows, st);
+    case 11:
+    case 12: return launch_mfma<12>(in, out, g, dA, W, H, nrows, st);
+  }
   const size_t lds = sizeof(double) * (size_t)(3 * W - 1);
   int blocks = nrows < 8192 ? nrows : 8192;
   prefilter_kernel<<<blocks, FDK_THREADS, lds, st>>>(in, out, g, dA, W, H, nrows);
