@@ -127,25 +127,30 @@ __device__ __forceinline__ float advance_rows(float pz, float dz, int z0) {
 // Cone row coordinates at the z-range starts: the reference steps
 // proj_z += U once per slice from z = 0 (CUDAmex_BP.cu:208-219), so the
 // value at z0 is the float running sum after z0 additions.  One thread per
-// (voxel column, view) runs the sum once and stores it at z0 = ZR, 2 ZR, ...,
-// which saves every range from replaying the additions before it.
+// (voxel column in the circle, view) runs the sum once and stores it at z0 = ZR,
+// 2 ZR, ..., which saves every range from replaying the additions before it.  A
+// wave takes a tile, whose place is then scalar arithmetic, and a grid row a
+// view: 301^2 x 211 x 250 views 162 -> 133 us against threads over (view, column)
+// outside the circle too; bound by the 540 MB it writes (4.1 TB/s).
 template <int ZR>
 __global__ __launch_bounds__(256) void bp_chain_kernel(BPKArgs a, float* chain) {
-  const size_t total = (size_t)a.ncols * a.nviews;
-  for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (size_t)gridDim.x * 256) {
-    const uint32_t col = (uint32_t)(t % a.ncols);
-    const int v = (int)(t / a.ncols);
-    int ix, iy;
-    tile_xy(col >> 6, col & 63u, a.tiles_x, a.super_, ix, iy);
-    if (ix >= a.W || iy >= a.W) continue;
-    const uint32_t hw = (uint32_t)a.W / 2u - 1u;
-    const float x = (float)ix - ((float)hw + 0.5f);
-    const float y = (float)iy - ((float)hw + 0.5f);
+  const uint32_t tile =
+      (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4u + (threadIdx.x >> 6)));
+  const uint32_t lane = threadIdx.x & 63u, col = tile * 64u + lane;
+  int ix, iy;
+  tile_xy(tile, lane, a.tiles_x, a.super_, ix, iy);
+  const uint32_t hw = (uint32_t)a.W / 2u - 1u;
+  const uint32_t dx = (uint32_t)ix - hw, dy = (uint32_t)iy - hw;
+  if (col >= a.ncols || ix >= a.W || iy >= a.W || !(dx * dx + dy * dy < hw * hw)) return;
+  const float x = (float)ix - ((float)hw + 0.5f);
+  const float y = (float)iy - ((float)hw + 0.5f);
+  for (int v = (int)blockIdx.y; v < a.nviews; v += (int)gridDim.y) {
     const float2 scv = a.sc[v];
     float U, py, pz, dz;
     bp_view_geom<GEOM_CONE>(x, y, scv.x, scv.y, a.SR, a.v0, hw, U, py, pz, dz);
     float* o = chain + (size_t)v * (a.nz - 1) * a.ncols + col;
     for (uint32_t r = 1; r < a.nz; ++r) {
+#pragma unroll
       for (int m = 0; m < ZR; ++m) pz = pz + dz;
       o[(size_t)(r - 1) * a.ncols] = pz;
     }
@@ -474,7 +479,7 @@ hipError_t launch_bp_chain(const float2* sc, int nviews, int W, int H, float sad
   k.nz = (uint32_t)((H + zr - 1) / zr);
   const uint32_t tpad = (k.tiles_x + k.super_ - 1) / k.super_ * k.super_;
   k.ncols = tpad * tpad * 64u;
-  const unsigned g = (unsigned)std::min<size_t>(((size_t)k.ncols * nviews + 255) / 256, 65536);
+  const dim3 g(k.ncols / 256u + (k.ncols % 256u != 0), (unsigned)std::min(nviews, 65535));
   if (zr == 64)
     bp_chain_kernel<64><<<g, 256, 0, st>>>(k, chain);
   else if (zr == 48)
