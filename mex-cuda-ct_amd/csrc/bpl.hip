@@ -8,7 +8,8 @@
 // columns by 1.2 ZW rows per view, each pixel some twenty times, so a workgroup
 // copies that window into LDS and gathers from there: two 8-byte LDS reads and
 // 13 VALU per update, no row clamp (the copy has a halo of edge rows).  Bound by
-// the VALU: 84% of its issue slots at 256^3, 14.7 per update with set-up.
+// LDS (89% busy at 384^3, 5.2 clocks for each 8-byte read of a wave, 4 at least)
+// and next the VALU (14.7 instructions an update with set-up).
 // Against the general kernel: 384^3 x 512 views 15.3 -> 11.6 ms, 256^3 x 360 3.90 ->
 // 2.38, 301^2 x 211 x 250 3.29 -> 2.35, 64^3 x 60 169 -> 98 us; never slower from 32^3
 // to 512^2 x 400.
@@ -75,9 +76,10 @@ struct ConeGeo {
 constexpr int kNoRows = (int)0x80000000;
 
 // ZR: slices per wave; CW: detector columns a stage holds per view; P: rows of
-// LDS per detector column, 4 modulo 64, so that neighbouring detector columns
-// start four banks apart and a wave's reads of up to 16 columns by 4 rows fall on
-// different banks.
+// LDS per detector column, an odd multiple of 4, so that neighbouring detector
+// columns start four banks apart and a wave's reads of up to 16 columns by 4 rows
+// fall on different banks (256^3 x 360 views: 196, 204, 212, 220, 228 rows 2.38-2.40
+// ms, 200 3.39, 208 5.48).
 template <int ZR, int CW, int P, bool LOADS>
 __global__ __launch_bounds__(256, 5) void bpl_kernel(BPLArgs a) {
   constexpr int ZW = 4 * ZR;
