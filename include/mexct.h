@@ -54,6 +54,7 @@ typedef struct mexct_opts {
   int32_t storage;  /* MEXCT_F32 (default, reference-exact), MEXCT_F16, MEXCT_BF16 */
   int32_t tv_steps; /* TVmin gradient steps; 0 -> 20 as CUDAmex_TVmin_3D.cu:221  */
   int32_t zrange;   /* BP z-voxels per thread: 32, 48 or 64; 0 -> chosen by H    */
+                    /* (the gathering kernel; the LDS ones choose their own)        */
   int32_t long_ray; /* F16/BF16 FP: rays of more samples than this are summed with  */
                     /* compensated (Kahan) summation; 0 -> 1024, < 0 -> never       */
   int32_t g3d_bp;   /* general-3D BP: MEXCT_G3D_BRICKS (0, default),                */
