@@ -175,14 +175,14 @@ __device__ __forceinline__ uint32_t load_bits(const u4v& q) { return q.x ^ q.y ^
 template <int GEOM, int ZR, typename S, bool SMALL, int RQ, bool ZC, bool LOADS = false>
 __global__ __launch_bounds__(64) void bp_kernel(BPKArgs a) {
   // Block order: the z-ranges one after another over the whole chip (a
-  // phase each), and in a phase (batch item, tile), each XCD taking a
-  // contiguous range.  Tiles go in super-tiles (row-major inside), so that
-  // the blocks an XCD runs together cover a compact region whose view
-  // footprints overlap; the voxels of one z-range project to a band of
+  // phase each), and in a phase (batch item, tile), the rows of super-tiles
+  // dealt to the XCDs in turn (xcd_deal).  Tiles go in super-tiles (row-major
+  // inside), so that the blocks that run together cover compact regions whose
+  // view footprints overlap; the voxels of one z-range project to a band of
   // detector rows whose row-paired copy stays in the memory-side cache
   // across the phase.
   const uint32_t zr = blockIdx.x / a.phase_blocks;
-  const uint32_t bl = xcd_remap(blockIdx.x - zr * a.phase_blocks, a.phase_blocks);
+  const uint32_t bl = xcd_deal(blockIdx.x - zr * a.phase_blocks, a.super_);
   if (bl >= a.phase_logical) return;
   const uint32_t tiles = a.item_blocks / a.nz;
   const uint32_t item = bl / tiles;  // batch item
@@ -415,7 +415,7 @@ template <int ZR, typename S, bool SMALL, int RQ, bool ZC>
 static void bp_dispatch_g(const BPKArgs& k0, int geom, hipStream_t st) {
   BPKArgs k = k0;  // z-ranges outermost (see bp_kernel)
   k.phase_logical = k.item_blocks / k.nz * (k.n_logical / k.item_blocks);
-  k.phase_blocks = padded_grid(k.phase_logical);
+  k.phase_blocks = xcd_deal_blocks(k.phase_logical, k.super_);
   const unsigned g = k.phase_blocks * k.nz;
   if (k.loads_only) {  // cone only (the host checks)
     bp_kernel<GEOM_CONE, ZR, S, SMALL, RQ, ZC, true><<<g, 64, 0, st>>>(k);

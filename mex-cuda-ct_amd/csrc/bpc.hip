@@ -119,9 +119,9 @@ __global__ __launch_bounds__(BPC_THREADS, 4) void bpc_kernel(BPCArgs a) {
   __shared__ __align__(16) char stage[bpc_stage_bytes(ZB, ES, CW)];
 
   // block order as bp_kernel's: the z-ranges one after another, tiles in
-  // super-tiles, a contiguous range per XCD
+  // super-tiles, their rows dealt to the XCDs
   const uint32_t zr = blockIdx.x / a.phase_blocks;
-  const uint32_t bl = xcd_remap(blockIdx.x - zr * a.phase_blocks, a.phase_blocks);
+  const uint32_t bl = xcd_deal(blockIdx.x - zr * a.phase_blocks, a.super_);
   if (bl >= a.phase_logical) return;
   const uint32_t tiles = a.item_blocks / a.nz;
   const uint32_t item = bl / tiles;
@@ -316,7 +316,7 @@ static hipError_t bpc_go(BPCArgs& k, int items, hipStream_t st) {
   if (per * k.nz * (uint64_t)items >= (1ull << 31)) return hipErrorInvalidValue;
   k.item_blocks = (uint32_t)(per * k.nz);
   k.phase_logical = (uint32_t)(per * items);
-  k.phase_blocks = (k.phase_logical + 7u) & ~7u;
+  k.phase_blocks = xcd_deal_blocks(k.phase_logical, k.super_);
   const unsigned g = k.phase_blocks * k.nz;
   // windows of 16 columns (40 KB of LDS for par, 44 for fan: three workgroups per
   // CU), 20 (fan sources nearer than about 4.5 radii: 52 KB, three) or 32 (76 KB,

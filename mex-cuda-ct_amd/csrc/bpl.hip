@@ -12,7 +12,7 @@
 // and next the VALU (14.7 instructions an update with set-up).
 // Against the general kernel: 384^3 x 512 views 15.3 -> 11.6 ms, 256^3 x 360 3.90 ->
 // 2.38, 301^2 x 211 x 250 3.29 -> 2.35, 64^3 x 60 169 -> 98 us; never slower from 32^3
-// to 512^2 x 400.
+// to 512^2 x 400 (with the tiles dealt to the XCDs, xcd_deal, 9.5, 2.2 and 2.0 ms).
 //
 // A 256-thread workgroup: wave w sums slices [w ZR, (w+1) ZR) of its 4 ZR, one
 // voxel column per lane, sums in registers over the views in the reference's
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256, 5) void bpl_kernel(BPLArgs a) {
 
   // block order as bp_kernel's
   const uint32_t zr = blockIdx.x / a.phase_blocks;
-  const uint32_t bl = xcd_remap(blockIdx.x - zr * a.phase_blocks, a.phase_blocks);
+  const uint32_t bl = xcd_deal(blockIdx.x - zr * a.phase_blocks, a.super_);
   if (bl >= a.phase_logical) return;
   const uint32_t tiles = a.item_blocks / a.nz;
   const uint32_t item = bl / tiles;
@@ -367,7 +367,7 @@ hipError_t launch_bpl(const BPLaunch& a, hipStream_t st) {
   if (per * k.nz * (uint64_t)items >= (1ull << 31)) return hipErrorInvalidValue;
   k.item_blocks = (uint32_t)(per * k.nz);
   k.phase_logical = (uint32_t)(per * items);
-  k.phase_blocks = (k.phase_logical + 7u) & ~7u;
+  k.phase_blocks = xcd_deal_blocks(k.phase_logical, k.super_);
   k.ncols = tpad * tpad * 64u;
   if (a.zr != p.zr && a.zr != 2 * p.zr) return hipErrorInvalidValue;
   k.cz = a.zr;
