@@ -246,4 +246,14 @@ inline uint32_t xcd_deal_blocks(uint32_t n, uint32_t group) {
   return ((n + group - 1u) / group + 7u) / 8u * 8u * group;
 }
 
+// Views per chunk of a projector's block order: at most 2^log2, the chunks as even
+// as they come, so that no XCD's range holds the empty places of a short last one:
+// parallel f32 128^3 x 180 views (12 chunks of 15, not 11 of 16 and one of 4) 379 ->
+// 368 us, 256^3 x 100 1.71 -> 1.61 ms, general-3D 256^3 x 100 4.26 -> 3.91 ms; the same
+// within 1% where the last chunk was full or one of many.
+inline uint32_t even_chunk(uint32_t nviews, uint32_t log2) {
+  const uint32_t n = (nviews + (1u << log2) - 1u) >> log2;
+  return n ? (nviews + n - 1u) / n : 1u;
+}
+
 }  // namespace mexct

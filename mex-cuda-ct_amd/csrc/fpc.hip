@@ -69,7 +69,7 @@ struct FPCArgs {
   uint32_t lz_log2;   // lanes per detector column
   uint32_t n_ug, n_vg, nv;
   int long_ray;
-  uint32_t vchunk_log2, item_blocks;
+  uint32_t vchunk, item_blocks;
   uint32_t phase_blocks, phase_logical;  // row groups one after another (see fpz.hip)
   uint64_t vol_stride, out_stride;
   float* const* outs;
@@ -282,10 +282,10 @@ __global__ __launch_bounds__(256) void fpc_kernel(FPCArgs a) {
   const uint32_t per = a.item_blocks / a.n_vg;
   const uint32_t item = bl / per;
   uint32_t rest = bl - item * per;
-  const uint32_t vw = rest & ((1u << a.vchunk_log2) - 1u);
-  rest >>= a.vchunk_log2;
+  const uint32_t vw = rest % a.vchunk;
+  rest /= a.vchunk;
   const uint32_t ug = rest % a.n_ug;
-  const uint32_t jv = ((rest / a.n_ug) << a.vchunk_log2) + vw;
+  const uint32_t jv = rest / a.n_ug * a.vchunk + vw;
   if (jv >= a.nv) return;
   const int lz = 1 << a.lz_log2;
   const int ix = (int)(ug << (8 - a.lz_log2)) + (int)(threadIdx.x >> a.lz_log2);
@@ -432,8 +432,7 @@ static unsigned set_grid(FPCArgs& k, int st_dt, int z, int vlog2, int items) {
   const int cols = 256 >> k.lz_log2;
   k.n_ug = (uint32_t)((k.W + cols - 1) / cols);
   k.n_vg = (uint32_t)((k.H + (1 << gl) - 1) >> gl);
-  k.vchunk_log2 = (uint32_t)vlog2;
-  const uint32_t c = 1u << vlog2;
+  const uint32_t c = k.vchunk = even_chunk(k.nv, (uint32_t)vlog2);
   const uint64_t nvp = (k.nv + c - 1) / c * (uint64_t)c;
   const uint64_t per = (uint64_t)k.n_ug * nvp;
   if (per * k.n_vg * (uint64_t)items >= (1ull << 31)) return 0;

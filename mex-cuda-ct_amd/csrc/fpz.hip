@@ -68,7 +68,7 @@ struct FPZArgs {
   uint32_t n_ug, n_vg, n_logical;
   uint32_t nv;  // views of the launch
   int long_ray;  // 2-byte storage: waves with a ray of more samples use compensated sums
-  uint32_t vchunk_log2;  // views per chunk of the block order: 1 << vchunk_log2
+  uint32_t vchunk;  // views per chunk of the block order
   uint32_t item_blocks;  // blocks of one batch item; n_logical = item_blocks * items
   // nonzero: the row groups run one after another, each in a phase of
   // phase_blocks grid blocks of which the first phase_logical work
@@ -504,7 +504,7 @@ __device__ __forceinline__ float march_z(__amdgpu_buffer_rsrc_t r, const FPZArgs
 // fold of each ray's taps (a measurement, not a projection).
 template <int GEOM, typename S, int EPI, int LAYOUT>
 __global__ __launch_bounds__(256) void fpz_kernel(FPZArgs a) {
-  // Block order: (batch item, chunk of 2^vchunk_log2 views, column group,
+  // Block order: (batch item, chunk of vchunk views, column group,
   // view in chunk), each XCD taking a contiguous range.  The blocks an XCD
   // runs together then march the same 4 detector columns of consecutive
   // views, whose rays lie within a few voxels of each other, so the volume
@@ -532,10 +532,10 @@ __global__ __launch_bounds__(256) void fpz_kernel(FPZArgs a) {
     b = bi / a.n_vg;
   }
   uint32_t rest = b;
-  const uint32_t vw = rest & ((1u << a.vchunk_log2) - 1u);
-  rest >>= a.vchunk_log2;
+  const uint32_t vw = rest % a.vchunk;
+  rest /= a.vchunk;
   const uint32_t ug = rest % a.n_ug;
-  const uint32_t jv = ((rest / a.n_ug) << a.vchunk_log2) + vw;
+  const uint32_t jv = rest / a.n_ug * a.vchunk + vw;
   if (jv >= a.nv) return;
   const int ix = (int)ug * 4 + (int)(threadIdx.x >> 6);
   const int iy = (int)vg * 64 + (int)(threadIdx.x & 63);
@@ -603,8 +603,7 @@ __global__ __launch_bounds__(256) void fpz_kernel(FPZArgs a) {
 
 // The block order's view chunk and the number of batch items.
 static void set_view_chunk(FPZArgs& k, uint32_t log2, uint32_t items) {
-  k.vchunk_log2 = log2;
-  const uint32_t c = 1u << log2;
+  const uint32_t c = k.vchunk = even_chunk(k.nv, log2);
   const uint32_t nvp = (k.nv + c - 1) / c * c;
   k.item_blocks = k.n_ug * k.n_vg * nvp;
   k.n_logical = k.item_blocks * items;
