@@ -1,7 +1,8 @@
-// bp.hip -- voxel-driven backprojectors (cone, fan with the source near the
-// circle, and the OSC dual backprojection with its update; parallel and other
-// fan scans take the column kernel, bpc.hip) and the general-3D ray-driven
-// scatter, for gfx950.
+// bp.hip -- voxel-driven backprojectors (cone in 2-byte storage, cone and fan
+// with the source near the circle, and the OSC dual backprojection with its
+// update; parallel and other fan scans take the column kernel, bpc.hip, other
+// f32 cone scans the LDS one, bpl.hip) and the general-3D ray-driven scatter,
+// for gfx950.
 //
 // Voxel-driven BP (CUDAmex_BP.cu:44-221): the reference launches one kernel
 // per view and read-modify-writes the whole volume each time (8 B per
