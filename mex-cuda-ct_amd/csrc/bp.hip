@@ -953,7 +953,16 @@ hipError_t launch_g3d_bp(const G3DBPLaunch& a, hipStream_t st) {
   k.pmax = a.pmax;
   k.gate = a.gate;
   if (k.n_logical == 0) return hipSuccess;
-  g3d_bp_kernel<<<padded_grid(k.n_logical), 256, 0, st>>>(k);
+  const int most = (int)std::min<uint64_t>((kThreads / 256 - 8) / k.tiles_per_view, INT32_MAX);
+  if (most == 0) return hipErrorInvalidValue;
+  for (int64_t v = 0; v < a.nviews; v += most) {
+    const int n = (int)std::min<int64_t>(most, a.nviews - v);
+    k.n_logical = k.tiles_per_view * (uint32_t)n;
+    g3d_bp_kernel<<<padded_grid(k.n_logical), 256, 0, st>>>(k);
+    k.sino += (size_t)n * a.W * a.H;
+    k.sc += n;
+    k.pts += n * k.pts_view_stride;
+  }
   return hipGetLastError();
 }
 

@@ -55,6 +55,7 @@ struct BPCArgs {
   float SR;
   uint32_t tiles_x, nz, super_;
   uint32_t item_blocks, phase_blocks, phase_logical;
+  uint32_t first;  // block of the order that this launch starts at
   uint64_t sino_stride, out_stride;
   float* const* outs;
 };
@@ -120,8 +121,9 @@ __global__ __launch_bounds__(BPC_THREADS, 4) void bpc_kernel(BPCArgs a) {
 
   // block order as bp_kernel's: the z-ranges one after another, tiles in
   // super-tiles, their rows dealt to the XCDs
-  const uint32_t zr = blockIdx.x / a.phase_blocks;
-  const uint32_t bl = xcd_deal(blockIdx.x - zr * a.phase_blocks, a.super_);
+  const uint32_t blk = blockIdx.x + a.first;
+  const uint32_t zr = blk / a.phase_blocks;
+  const uint32_t bl = xcd_deal(blk - zr * a.phase_blocks, a.super_);
   if (bl >= a.phase_logical) return;
   const uint32_t tiles = a.item_blocks / a.nz;
   const uint32_t item = bl / tiles;
@@ -317,17 +319,23 @@ static hipError_t bpc_go(BPCArgs& k, int items, hipStream_t st) {
   k.item_blocks = (uint32_t)(per * k.nz);
   k.phase_logical = (uint32_t)(per * items);
   k.phase_blocks = xcd_deal_blocks(k.phase_logical, k.super_);
-  const unsigned g = k.phase_blocks * k.nz;
+  const uint64_t blocks = (uint64_t)k.phase_blocks * k.nz;
+  if (blocks >= (1ull << 32)) return hipErrorInvalidValue;
   // windows of 16 columns (40 KB of LDS for par, 44 for fan: three workgroups per
   // CU), 20 (fan sources nearer than about 4.5 radii: 52 KB, three) or 32 (76 KB,
   // two)
-  if (k.cw <= 16)
-    bpc_kernel<GEOM, S, ZB, 16><<<g, BPC_THREADS, 0, st>>>(k);
-  else if constexpr (GEOM == GEOM_FAN) {
-    if (k.cw <= 20)
-      bpc_kernel<GEOM, S, ZB, 20><<<g, BPC_THREADS, 0, st>>>(k);
-    else
-      bpc_kernel<GEOM, S, ZB, 32><<<g, BPC_THREADS, 0, st>>>(k);
+  constexpr uint64_t most = kThreads / BPC_THREADS - 8;  // a multiple of 8 (the XCDs)
+  for (uint64_t b = 0; b < blocks; b += most) {
+    k.first = (uint32_t)b;
+    const unsigned g = (unsigned)std::min(most, blocks - b);
+    if (k.cw <= 16)
+      bpc_kernel<GEOM, S, ZB, 16><<<g, BPC_THREADS, 0, st>>>(k);
+    else if constexpr (GEOM == GEOM_FAN) {
+      if (k.cw <= 20)
+        bpc_kernel<GEOM, S, ZB, 20><<<g, BPC_THREADS, 0, st>>>(k);
+      else
+        bpc_kernel<GEOM, S, ZB, 32><<<g, BPC_THREADS, 0, st>>>(k);
+    }
   }
   return hipGetLastError();
 }

@@ -364,7 +364,8 @@ hipError_t launch_bpl(const BPLaunch& a, hipStream_t st) {
   k.super_ = a.super_ > 0 ? (uint32_t)a.super_ : 4u;
   const uint32_t tpad = (k.tiles_x + k.super_ - 1) / k.super_ * k.super_;
   const uint64_t per = (uint64_t)tpad * tpad;
-  if (per * k.nz * (uint64_t)items >= (1ull << 31)) return hipErrorInvalidValue;
+  // (a block writes 8 KB or more: the memory is full before a launch is too long)
+  if (per * k.nz * (uint64_t)items >= kThreads / 256 - (1u << 16)) return hipErrorInvalidValue;
   k.item_blocks = (uint32_t)(per * k.nz);
   k.phase_logical = (uint32_t)(per * items);
   k.phase_blocks = xcd_deal_blocks(k.phase_logical, k.super_);

@@ -15,6 +15,8 @@
 // Staging also applies, in the reference's order, FBP_recon's
 // -log(post./pre) with NaN/Inf -> 0 (FBP_recon.m:26-28) when a post array
 // is given, and the Parker window after the cosine weight (:60).
+#include <algorithm>
+
 #include "common.h"
 #include "internal.h"
 
@@ -90,13 +92,13 @@ __global__ __launch_bounds__(FDK_THREADS) void prefilter_kernel(
 template <int MR, int NT>
 __global__ __launch_bounds__(FDK_THREADS, 2) void prefilter_mfma_kernel(
     FilterIn in, float* __restrict__ out, const double* __restrict__ g,
-    const float* __restrict__ dA, int W, int H, int nrows) {
+    const float* __restrict__ dA, int W, int H, int nrows, int first) {
   typedef double d4v __attribute__((ext_vector_type(4)));
   extern __shared__ double lds[];
   const int Kp = (W + 3) & ~3, XS = Kp | 1, GL = 64 * NT + Kp;
   double* const gs = lds;  // gs[Kp - 1 + d] = tap d
   float* const xs = (float*)(lds + GL);
-  const int row0 = (int)blockIdx.x * (16 * MR);
+  const int row0 = first + (int)blockIdx.x * (16 * MR);
   for (int i = threadIdx.x; i < GL; i += FDK_THREADS) {
     const int k = i - Kp + W;
     gs[i] = k >= 0 && k < 2 * W - 1 ? g[k] : 0.0;
@@ -162,12 +164,16 @@ static hipError_t launch_mfma(const FilterIn& in, float* out, const double* g, c
   const int Kp = (W + 3) & ~3;
   const size_t taps = sizeof(double) * (size_t)(64 * NT + Kp);
   // 32 rows per workgroup where that still gives two to every CU
-  if (nrows >= 32 * 512)
-    prefilter_mfma_kernel<2, NT><<<(nrows + 31) / 32, FDK_THREADS, taps + sizeof(float) * 32 * (size_t)(Kp | 1), st>>>(
-        in, out, g, dA, W, H, nrows);
-  else
+  if (nrows >= 32 * 512) {
+    constexpr int most = (int)(kThreads / FDK_THREADS - 8) * 32;  // rows per launch
+    for (int64_t r = 0; r < nrows; r += most)
+      prefilter_mfma_kernel<2, NT><<<(unsigned)((std::min<int64_t>(most, nrows - r) + 31) / 32), FDK_THREADS,
+                                     taps + sizeof(float) * 32 * (size_t)(Kp | 1), st>>>(
+          in, out, g, dA, W, H, nrows, (int)r);
+  } else {
     prefilter_mfma_kernel<1, NT><<<(nrows + 15) / 16, FDK_THREADS, taps + sizeof(float) * 16 * (size_t)(Kp | 1), st>>>(
-        in, out, g, dA, W, H, nrows);
+        in, out, g, dA, W, H, nrows, 0);
+  }
   return hipGetLastError();
 }
 

@@ -9,6 +9,8 @@
 // workgroup id is remapped so each XCD walks a contiguous run of patches.
 // Each sample is an 8-tap trilinear fetch: four pair loads of (i, i+1)
 // along x, lerps x, then y, then z (ray setup and clip in ray.h).
+#include <algorithm>
+
 #include "common.h"
 #include "internal.h"
 #include "ray.h"
@@ -146,12 +148,21 @@ hipError_t launch_fp(const FPLaunch& a, hipStream_t st) {
   k.pts = a.pts;
   k.pts_view_stride = a.pts_view_stride;
   if (k.n_logical == 0) return hipSuccess;
-  if (a.st_dt == 0)
-    fp_dispatch<float>(k, a.geom, st);
-  else if (a.st_dt == 1)
-    fp_dispatch<_Float16>(k, a.geom, st);
-  else
-    fp_dispatch<bf16_t>(k, a.geom, st);
+  const int most = (int)std::min<uint64_t>((kThreads / 256 - 8) / k.tiles_per_view, INT32_MAX);
+  if (most == 0) return hipErrorInvalidValue;
+  for (int64_t v = 0; v < a.nviews; v += most) {
+    const int n = (int)std::min<int64_t>(most, a.nviews - v);
+    k.n_logical = k.tiles_per_view * (uint32_t)n;
+    if (a.st_dt == 0)
+      fp_dispatch<float>(k, a.geom, st);
+    else if (a.st_dt == 1)
+      fp_dispatch<_Float16>(k, a.geom, st);
+    else
+      fp_dispatch<bf16_t>(k, a.geom, st);
+    k.out += (size_t)n * a.W * a.H;
+    k.sc += n;
+    if (k.pts) k.pts += n * k.pts_view_stride;
+  }
   return hipGetLastError();
 }
 

@@ -426,6 +426,7 @@ static int pick_rows(const FPCArgs& k, bool osc2, int items) {
   return (uint64_t)k.W * k.H * k.nv * (uint64_t)items >= waves * 256 ? 4 : 1;
 }
 
+// The launch's block order and grid; 0 past kThreads.
 static unsigned set_grid(FPCArgs& k, int st_dt, int z, int vlog2, int items) {
   const uint32_t gl = group_log2(k.H, st_dt);
   k.lz_log2 = gl - (z == 4 ? 2 : 0);
@@ -435,7 +436,7 @@ static unsigned set_grid(FPCArgs& k, int st_dt, int z, int vlog2, int items) {
   const uint32_t c = k.vchunk = even_chunk(k.nv, (uint32_t)vlog2);
   const uint64_t nvp = (k.nv + c - 1) / c * (uint64_t)c;
   const uint64_t per = (uint64_t)k.n_ug * nvp;
-  if (per * k.n_vg * (uint64_t)items >= (1ull << 31)) return 0;
+  if (((per * items + 7) & ~7ull) * k.n_vg >= kThreads / 256) return 0;
   k.item_blocks = (uint32_t)(per * k.n_vg);
   k.phase_logical = (uint32_t)(per * items);
   k.phase_blocks = (k.phase_logical + 7u) & ~7u;
@@ -459,11 +460,26 @@ template <int EPI>
 static hipError_t fpc_dispatch_s(FPCArgs& k, int st_dt, int geom, int vlog2, int items,
                                  hipStream_t st) {
   const int z = pick_rows(k, EPI == 1 && st_dt != 0, items);
-  const unsigned g = set_grid(k, st_dt, z, vlog2, items);
-  if (g == 0) return hipErrorInvalidValue;
-  if (st_dt == 0) return fpc_dispatch<float, EPI>(k, geom, z, g, st);
-  if (st_dt == 1) return fpc_dispatch<_Float16, EPI>(k, geom, z, g, st);
-  return fpc_dispatch<bf16_t, EPI>(k, geom, z, g, st);
+  const uint32_t nv = k.nv;
+  uint32_t most = nv;  // views per launch
+  if (set_grid(k, st_dt, z, vlog2, items) == 0) {
+    // past kThreads: half of them at a time, which leaves room for the padding
+    if (EPI == 1) return hipErrorInvalidValue;  // (its copies are indexed by the launch's views)
+    most = (uint32_t)std::max<uint64_t>(1, kThreads / 512 / ((uint64_t)k.n_ug * k.n_vg * items));
+  }
+  hipError_t e = hipSuccess;
+  for (uint32_t v = 0; v < nv && e == hipSuccess; v += most) {
+    if (most < nv) {
+      k.first = (int)v;
+      k.nv = std::min(most, nv - v);
+    }
+    const unsigned g = set_grid(k, st_dt, z, vlog2, items);
+    if (g == 0) return hipErrorInvalidValue;
+    e = st_dt == 0   ? fpc_dispatch<float, EPI>(k, geom, z, g, st)
+        : st_dt == 1 ? fpc_dispatch<_Float16, EPI>(k, geom, z, g, st)
+                     : fpc_dispatch<bf16_t, EPI>(k, geom, z, g, st);
+  }
+  return e;
 }
 
 hipError_t launch_fpc(const FPZLaunch& a, hipStream_t st) {

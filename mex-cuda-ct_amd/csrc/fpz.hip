@@ -33,6 +33,8 @@
 // the plain one, which MI355X's HBM holds easily; volumes whose copy would
 // pass 4 GiB use PLAIN.
 
+#include <algorithm>
+
 #include "common.h"
 #include "internal.h"
 #include "ray.h"
@@ -730,29 +732,38 @@ hipError_t launch_fpz(const FPZLaunch& a, hipStream_t st) {
   if (a.long_ray != 0) k.long_ray = a.long_ray;
   if (a.geom == GEOM_G3D) k.rows = a.H;  // every detector row is a ray
   const int items = a.items > 0 ? a.items : 1;
-  set_view_chunk(k,
-                 a.vchunk_log2 >= 0          ? (uint32_t)a.vchunk_log2
-                 : a.geom == GEOM_G3D ? kViewChunkLog2G3D
-                                      : kViewChunkLog2,
-                 (uint32_t)items);
+  const uint32_t vlog2 = a.vchunk_log2 >= 0          ? (uint32_t)a.vchunk_log2
+                         : a.geom == GEOM_G3D ? kViewChunkLog2G3D
+                                              : kViewChunkLog2;
   k.vol_stride = a.vol_stride;
   k.out_stride = a.out_stride;
   k.outs = a.outs;
-  if ((uint64_t)k.item_blocks * (uint64_t)items >= (1ull << 31)) return hipErrorInvalidValue;
-  if (k.n_logical == 0) return hipSuccess;
-  if (a.loads_only) {
-    const hipError_t e = a.st_dt == 0   ? fpz_loads_dispatch<float>(k, a.geom, a.layout, st)
-                         : a.st_dt == 1 ? fpz_loads_dispatch<_Float16>(k, a.geom, a.layout, st)
-                                        : fpz_loads_dispatch<bf16_t>(k, a.geom, a.layout, st);
-    return e != hipSuccess ? e : hipGetLastError();
+  if (k.nv == 0) return hipSuccess;
+  // past kThreads: whole views, half of the threads at a time, which leaves room
+  // for the padding of the block order
+  const uint64_t per_view = (uint64_t)k.n_ug * k.n_vg * (uint64_t)items;
+  const bool fits = per_view * ((uint64_t)k.nv + (1u << vlog2)) + 8u * k.n_vg < kThreads / 256;
+  const uint32_t most = fits ? k.nv : (uint32_t)std::max<uint64_t>(1, kThreads / 512 / per_view);
+  for (uint32_t v = 0; v < (uint32_t)a.nviews; v += most) {
+    k.first = (int)v;
+    k.nv = std::min(most, (uint32_t)a.nviews - v);
+    set_view_chunk(k, vlog2, (uint32_t)items);
+    if (k.item_blocks * (uint64_t)items + 8u * k.n_vg >= kThreads / 256) return hipErrorInvalidValue;
+    hipError_t e = hipSuccess;
+    if (a.loads_only)
+      e = a.st_dt == 0   ? fpz_loads_dispatch<float>(k, a.geom, a.layout, st)
+          : a.st_dt == 1 ? fpz_loads_dispatch<_Float16>(k, a.geom, a.layout, st)
+                         : fpz_loads_dispatch<bf16_t>(k, a.geom, a.layout, st);
+    else if (a.st_dt == 0)
+      fpz_dispatch<0, float>(k, a.geom, a.layout, st);
+    else if (a.st_dt == 1)
+      fpz_dispatch<0, _Float16>(k, a.geom, a.layout, st);
+    else
+      fpz_dispatch<0, bf16_t>(k, a.geom, a.layout, st);
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
-  if (a.st_dt == 0)
-    fpz_dispatch<0, float>(k, a.geom, a.layout, st);
-  else if (a.st_dt == 1)
-    fpz_dispatch<0, _Float16>(k, a.geom, a.layout, st);
-  else
-    fpz_dispatch<0, bf16_t>(k, a.geom, a.layout, st);
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 hipError_t launch_osc_fp(const OSCFPLaunch& a, hipStream_t st) {
@@ -769,6 +780,7 @@ hipError_t launch_osc_fp(const OSCFPLaunch& a, hipStream_t st) {
   k.PV = (a.W + 2 * HALO) * (a.H + 3);  // pairs per view: rows -2 .. H
   if (a.long_ray != 0) k.long_ray = a.long_ray;
   if (k.n_logical == 0) return hipSuccess;
+  if (k.n_logical >= kThreads / 256 - 8) return hipErrorInvalidValue;
   if (a.st_dt == 0)
     fpz_dispatch<1, float>(k, a.geom, a.layout, st);
   else if (a.st_dt == 1)

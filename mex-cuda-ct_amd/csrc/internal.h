@@ -11,6 +11,10 @@ struct mexct_opts;
 
 namespace mexct {
 
+// A grid dimension of 2^32 threads or more runs short without an error: launches of
+// more (whatever the geometry admits) go as several, kThreads / block threads at most.
+constexpr uint64_t kThreads = (uint64_t)1 << 32;
+
 // ---- storage conversion + halo padding (pad.hip)
 // 3D: in [nx,ny,nz] (dtype in_dt) -> out [nx+4, ny+4, nz+4] of storage st_dt.
 hipError_t launch_pad3(const void* in, int in_dt, void* out, int st_dt, int nx, int ny, int nz,

@@ -153,7 +153,8 @@ struct TVStep {
   int64_t sy_out, sz_out;
   float* gout;  // dense
   int nx, ny, nz, zc;  // zc: slices per workgroup
-  uint32_t gx, gy, n;  // workgroups along x, along y, of the launch
+  uint32_t gx, gy, n;  // workgroups along x, along y, in all
+  uint32_t first, padded;  // that this launch starts at; n in whole turns of the XCDs
   const double* pin;   // previous partials, np of them
   size_t np;
   const float* a_dev;  // non-null: a is there (np past kTVOwnSum)
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(256) void tv_step_kernel(TVStep t) {
   __shared__ float a_sh;
   // x fastest, then y, then z, each XCD a contiguous range: the rows and slices
   // that neighbouring workgroups both load come from one L2
-  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t b = xcd_remap(blockIdx.x + t.first, t.padded);
   if (b >= t.n) return;
   const int bx = (int)(b % t.gx), by = (int)(b / t.gx % t.gy), bz = (int)(b / t.gx / t.gy);
   const int li = (int)threadIdx.x & (LW - 1), rg = (int)threadIdx.x / LW;
@@ -356,12 +357,17 @@ size_t tv_partials_count(int nx, int ny, int nz) {
 }
 
 template <int LW, int RY>
-static void tv_step_go(const TVStep& t, hipStream_t st) {
-  const unsigned g = (t.n + 7u) & ~7u;
-  if (t.gin)
-    tv_step_kernel<LW, RY, false><<<g, 256, 0, st>>>(t);
-  else
-    tv_step_kernel<LW, RY, true><<<g, 256, 0, st>>>(t);
+static void tv_step_go(const TVStep& t0, hipStream_t st) {
+  TVStep t = t0;
+  t.padded = (t.n + 7u) & ~7u;
+  constexpr uint32_t most = (uint32_t)(kThreads / 256) - 8;
+  for (t.first = 0; t.first < t.padded; t.first += most) {
+    const unsigned g = std::min(most, t.padded - t.first);
+    if (t.gin)
+      tv_step_kernel<LW, RY, false><<<g, 256, 0, st>>>(t);
+    else
+      tv_step_kernel<LW, RY, true><<<g, 256, 0, st>>>(t);
+  }
 }
 static void tv_step(const TVStep& t, const TVPlan& p, hipStream_t st) {
   if (p.lw == 32)
