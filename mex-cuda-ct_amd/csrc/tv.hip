@@ -95,14 +95,16 @@ __device__ __forceinline__ float tv_sqrt(float s) {
   const float g = s * y, h = 0.5f * y;
   return __builtin_fmaf(__builtin_fmaf(-g, g, s), h, g);
 }
-// 1 / d to within an ulp, Newton-Raphson from the hardware reciprocal
+// 1 / d, Newton-Raphson from the hardware reciprocal: the IEEE quotient for every
+// float d in [2^-21, 2^63), and the same mantissa in each binade (all compared)
 __device__ __forceinline__ float tv_rcp(float d) {
   const float r = __builtin_amdgcn_rcpf(d);
   return __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
 }
-// n / d by Markstein's residual correction of n r, r = tv_rcp(d), for n = 0 or
-// |n| >= 2^-100 (the residual is then exact): equal to the IEEE quotient in 2e10
-// random pairs (d in [2^-20, 2^25], |n| in [2^-67, 2^-4])
+// n / d by Markstein's residual correction of n r, r = tv_rcp(d): the IEEE quotient
+// of every pair of mantissas (all 2^46 compared), so of every n and d whose quotient
+// and residual are normal or exact: n = 0, or |n| >= 2^-99 and d <= 2^25 (the
+// quotient is then 2^-124 at least; below 2^-126 it would be rounded twice)
 __device__ __forceinline__ float tv_div(float n, float d, float r) {
   const float q = n * r;
   return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
@@ -110,8 +112,9 @@ __device__ __forceinline__ float tv_div(float n, float d, float r) {
 
 constexpr float kTVEps = (float)1.0e-6;
 
-// FAST: every voxel value is 0 or between 2^-76 and 2^58 in magnitude, so that
-// the differences are 0 or at least 2^-100 (the ulp of 2^-76) and s1 below 2^120.
+// FAST: every voxel value is 0 or between 2^-76 and 2^22 in magnitude, so that
+// the differences are 0 or between 2^-99 (the ulp of 2^-76) and 2^23, and the
+// denominators below 2^25.
 template <bool FAST>
 __device__ __forceinline__ TVQ tv_quotients(float dx, float dy, float dz) {
   const float xx = dx * dx, yy = dy * dy, zz = dz * dz;
@@ -236,7 +239,7 @@ __global__ __launch_bounds__(256) void tv_step_kernel(TVStep t) {
       hi = max(hi, m);
     }
     return __builtin_amdgcn_ballot_w64(lo < (__float_as_uint(0x1p-76f) << 1) - 1u ||
-                                       hi > __float_as_uint(0x1p58f) << 1) != 0;
+                                       hi > __float_as_uint(0x1p22f) << 1) != 0;
   };
   float cur[RY + 2], prev[RY + 2], part[RY];
   double sq = 0.0;
