@@ -68,7 +68,12 @@ typedef struct mexct_ctx mexct_ctx;
 int mexct_ctx_create(mexct_ctx** ctx, int device, void* stream);
 int mexct_ctx_destroy(mexct_ctx* ctx);
 int mexct_ctx_sync(mexct_ctx* ctx);
-/* bytes of device workspace currently held by the context */
+/* bytes of device workspace currently held by the context: what its calls so far
+ * needed, kept until the context is destroyed.  The TV minimisation holds 4 bytes a
+ * voxel, and 8 more that only make it faster: those are taken where they are at
+ * most a quarter of the free memory (volumes of up to 16 GiB, not under stream capture), and freed
+ * when another allocation of the context would fail.  A captured call may be
+ * replayed until the context allocates again. */
 int64_t mexct_ctx_workspace_bytes(const mexct_ctx* ctx);
 const char* mexct_last_error(void);
 int mexct_version(void);

@@ -209,10 +209,8 @@ struct mexct_ctx {
         b.cap = 0;
       }
       size_t cap = (bytes + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
-      hipError_t e = hipMalloc(&b.p, cap);
+      const hipError_t e = alloc(&b.p, cap);
       if (e != hipSuccess) {
-        (void)hipGetLastError();
-        b.p = nullptr;
         return fail(MEXCT_ENOMEM, "device allocation of %zu bytes failed (%s)", cap,
                     hipGetErrorString(e));
       }
@@ -222,15 +220,65 @@ struct mexct_ctx {
     return MEXCT_OK;
   }
 
-  int drop(int slot) {
-    Buf& b = ws[slot];
-    if (b.p) {
-      HIPCHK(hipStreamSynchronize(stream));
-      HIPCHK(hipFree(b.p));
-      b.p = nullptr;
-      b.cap = 0;
+  // The second volumes of the TV step only make it faster: they are given back when
+  // another allocation of the context does not fit beside them.
+  bool drop_spare() {
+    bool any = false;
+    for (int slot : {WS_TVG2, WS_TVX2}) {
+      Buf& b = ws[slot];
+      if (!b.p) continue;
+      if (hipStreamSynchronize(stream) != hipSuccess || hipFree(b.p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+      b = Buf{};
+      any = true;
     }
-    return MEXCT_OK;
+    return any;
+  }
+  hipError_t alloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && drop_spare()) {
+      (void)hipGetLastError();
+      e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      *p = nullptr;
+    }
+    return e;
+  }
+  // Both second volumes of `bytes` each; false, with no error, under capture (an
+  // allocation would end it) and where they would take more than a quarter of the
+  // free memory.
+  bool get_spare(size_t bytes, void** g2, void** x2) {
+    Buf &a = ws[WS_TVG2], &b = ws[WS_TVX2];
+    if (a.cap < bytes || b.cap < bytes) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+      }
+      (void)drop_spare();
+      const size_t cap = (bytes + ((size_t)2 << 20) - 1) & ~(((size_t)2 << 20) - 1);
+      size_t avail = 0, total = 0;
+      if (hipMemGetInfo(&avail, &total) != hipSuccess || avail / 8 < cap) {
+        (void)hipGetLastError();
+        return false;
+      }
+      for (Buf* s : {&a, &b}) {
+        if (hipMalloc(&s->p, cap) != hipSuccess) {
+          (void)hipGetLastError();
+          s->p = nullptr;
+          (void)drop_spare();
+          return false;
+        }
+        s->cap = cap;
+      }
+    }
+    *g2 = a.p;
+    *x2 = b.p;
+    return true;
   }
 
   // Stage `bytes` of host data through pinned memory into device memory.
@@ -268,7 +316,7 @@ struct mexct_ctx {
       }
       sc_dev = nullptr;
       size_t cap = std::max<size_t>(h.size(), 1024);
-      HIPCHK(hipMalloc((void**)&sc_dev, cap * sizeof(float2)));
+      HIPCHK(alloc((void**)&sc_dev, cap * sizeof(float2)));
       sc_cap = cap;
     }
     if (!h.empty()) RC(upload(sc_dev, h.data(), h.size() * sizeof(float2)));
@@ -1485,15 +1533,11 @@ int tv_run(mexct_ctx* c, Vol3 x, const float* c_dev, float cc, int steps) {
   RC(c->get(WS_PARTIALS, tv_partials_count(x.nx, x.ny, x.nz) * 8, &pp));
   RC(c->get(WS_SCALARS, 256, &sp));
   // two volumes more for steps that carry the update along; a volume above
-  // 16 GiB (2^32 voxels), or memory that does not hold them, takes an update pass per step
+  // 16 GiB (2^32 voxels), or one that get_spare refuses, takes an update pass per step
   TVWork w;
-  if (steps > 1 && vb <= ((size_t)16 << 30) && c->get(WS_TVG2, vb, &g2) == MEXCT_OK) {
-    if (c->get(WS_TVX2, vb, &x2) == MEXCT_OK) {
-      w.g2 = (float*)g2;
-      w.x2 = (float*)x2;
-    } else {
-      RC(c->drop(WS_TVG2));
-    }
+  if (steps > 1 && vb <= ((size_t)16 << 30) && c->get_spare(vb, &g2, &x2)) {
+    w.g2 = (float*)g2;
+    w.x2 = (float*)x2;
   }
   w.g = (float*)gp;
   w.partials = (double*)pp;
