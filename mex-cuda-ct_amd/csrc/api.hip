@@ -717,8 +717,9 @@ size_t op_workspace_bytes(int op, int geom, int st, int64_t W, int64_t H, int64_
     const int zh = bp_row_halo(W, H, geom, sad, rows, st, &zc);
     size_t vb = (size_t)(W + 4) * (H + 2 * zh - 1) * rows * es;
     int lchain = 0;
-    const bool lds = geom == GEOM_CONE && st == MEXCT_F32 &&
-                     bpl_shape(W, H, sad, (int)nitems, nullptr, nullptr, &lchain, &vb);
+    // a batch of this request may choose another slice count, or the general kernel,
+    // whose copy is then the most
+    const bool lds = geom == GEOM_CONE && st == MEXCT_F32 && bpl_bound(W, H, sad, &lchain, &vb);
     if (!lds) (void)bpc_shape(W, H, geom, sad, st, nullptr, &vb);
     b += slot(vb * n * nitems);
     if (geom == 2 && st == MEXCT_F32) {

@@ -270,7 +270,15 @@ struct BPLPlan {
   int zr, p, cw, rw, zt, pv;
   double umax;
 };
-static bool bpl_plan(int64_t W, int64_t H, float sad, int items, BPLPlan* out) {
+// every wave's own start at 32 slices per wave, every other's below; 64 apart at 32
+// the same within 2% (2419 against 2374 us at 256^3 x 360; at 384^3 x 512, where
+// the scratch holds a third of the views, 11.4-11.7 against 11.6-11.9 ms)
+static int bpl_chain_slices(int zr) { return zr == 24 ? 48 : 32; }
+
+// pv_max, chain_min: if not null, the most rows of the copy and the least chain
+// spacing of the slice counts that a batch of some size takes.
+static bool bpl_plan(int64_t W, int64_t H, float sad, int items, BPLPlan* out, int* pv_max = nullptr,
+                     int* chain_min = nullptr) {
   // the running sum stays within a quarter row of its line up to 2048 rows
   if (W < 4 || W > 4096 || H < 1 || H > 2048) return false;
   const double r = (double)(W / 2 - 1) + 1.0, S = (double)sad, v0 = (H - 1) / 2.0;
@@ -291,6 +299,11 @@ static bool bpl_plan(int64_t W, int64_t H, float sad, int items, BPLPlan* out) {
     const int rw = ((int)std::ceil((zw - 1) * U + vm * dU) + 8 + 3) / 4 * 4;
     const int p = zr == 32 ? 196 : rw <= 132 || zr == 16 ? 132 : 196;
     if (rw > p) continue;
+    const int zt = ((int)std::ceil(v0 * (U - 1.0)) + 4 + 3) / 4 * 4;
+    const int top = (int)std::ceil(v0 + ((double)hp - v0) * U) + 4;
+    const int pv = std::max((zt + std::max(top, (int)H) + 3) / 4 * 4, rw);
+    if (pv_max) *pv_max = std::max(*pv_max, pv);
+    if (chain_min) *chain_min = std::min(*chain_min, bpl_chain_slices(zr));
     // A wave's time is its slices and about 8 more of set-up; a CU's, the waves
     // with slices to sum over the rate that so many in flight reach (one
     // workgroup about half, four all of it), and never less than one workgroup's.
@@ -305,14 +318,17 @@ static bool bpl_plan(int64_t W, int64_t H, float sad, int items, BPLPlan* out) {
       out->zr = zr;
       out->p = p;
       out->rw = rw;
-      out->zt = ((int)std::ceil(v0 * (U - 1.0)) + 4 + 3) / 4 * 4;
-      const int top = (int)std::ceil(v0 + ((double)hp - v0) * U) + 4;
-      out->pv = std::max((out->zt + std::max(top, (int)H) + 3) / 4 * 4, rw);
+      out->zt = zt;
+      out->pv = pv;
     }
   }
   out->cw = (int)cols;
   out->umax = U * 1.0001;
-  // no larger than the general kernel's row-paired copy
+  // No larger than the general kernel's row-paired copy.  (Taking the next slice count
+  // that fits instead pads the slices by more than it gains at few views or little
+  // more than one workgroup's slices: one by one 351^2 x 60 x 100 views 442 -> 474 us, but
+  // 251^2 x 67 x 100 385 -> 288; 16 scans of 82^2 x 58 at a time, 8 views 113 -> 152 us, 200
+  // views 855 -> 901, but of 173^2 x 40, 200 views 2.89 -> 2.28 ms.)
   return least < 1e300 && out->pv <= 2 * (H + 3);
 }
 
@@ -322,11 +338,17 @@ bool bpl_shape(int64_t W, int64_t H, float sad, int items, int* zt, int* pv, int
   if (!bpl_plan(W, H, sad, items, &p)) return false;
   if (zt) *zt = p.zt;
   if (pv) *pv = p.pv;
-  // every wave's own start at 32 slices per wave, every other's below; 64 apart
-  // at 32 the same within 2% (2419 against 2374 us at 256^3 x 360; at 384^3 x 512, where
-  // the scratch holds a third of the views, 11.4-11.7 against 11.6-11.9 ms)
-  if (chain_slices) *chain_slices = p.zr == 24 ? 48 : 32;
+  if (chain_slices) *chain_slices = bpl_chain_slices(p.zr);
   if (view_bytes) *view_bytes = (size_t)(W + 2 * HALO) * p.pv * 4;
+  return true;
+}
+
+bool bpl_bound(int64_t W, int64_t H, float sad, int* chain_slices, size_t* view_bytes) {
+  BPLPlan p;
+  int pv = 0;
+  *chain_slices = 64;
+  if (!bpl_plan(W, H, sad, 1, &p, &pv, chain_slices) || pv > 2 * (H + 3)) return false;
+  *view_bytes = (size_t)(W + 2 * HALO) * pv * 4;
   return true;
 }
 

@@ -209,6 +209,9 @@ hipError_t launch_bp_chain(const float2* sc, int nviews, int W, int H, float sad
 // chain_slices; rows, zh, zclamp unused).
 bool bpl_shape(int64_t W, int64_t H, float sad, int items, int* zt, int* pv, int* chain_slices,
                size_t* view_bytes);
+// Whether a batch of any size takes it, and then the most bytes of its copies and the
+// least chain spacing, for which the scratch is the largest.
+bool bpl_bound(int64_t W, int64_t H, float sad, int* chain_slices, size_t* view_bytes);
 hipError_t launch_bpl(const BPLaunch& a, hipStream_t st);
 // floats of BP chain scratch per view (cone f32, z-range zr, super-tile side)
 size_t bp_chain_floats_per_view(int W, int H, int zr, int super_);
