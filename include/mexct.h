@@ -125,7 +125,8 @@ int mexct_bp_batch_dev(mexct_ctx* ctx, const void* sinos, int32_t sino_dtype, in
  * No counterpart in the reference.  The FP and BP kernels' block order (FP:
  * views per chunk; BP: super-tile side, and the z-range for FP32 storage
  * unless opts fixes it) is tuned per problem shape (operator, geometry,
- * storage, W, H, nProj; any batch count): the tuning call of a shape times
+ * storage, W, H, nProj; any batch count), for each kernel that its calls take
+ * (a near source takes another one than a far one): the tuning call of a shape times
  * every candidate once on its first 128 (FP) or 32 (BP) views, keeps the
  * fastest for the
  * process and runs the call with it.  Candidates write identical bits.
@@ -134,7 +135,8 @@ int mexct_bp_batch_dev(mexct_ctx* ctx, const void* sinos, int32_t sino_dtype, in
  * built-in choices).  A context's own setting (-1: follow the global one)
  * overrides.  mexct_tuned_config fills cfg[4] = {found, FP views-per-chunk
  * log2 or BP super-tile side, BP z-range, the winner's time on the tuning
- * views in microseconds}. */
+ * views in microseconds}; of a shape tuned for several kernels, the one that
+ * far sources take. */
 int mexct_set_autotune(int32_t mode);
 int mexct_ctx_set_autotune(mexct_ctx* ctx, int32_t mode);
 int mexct_tuned_config(int32_t op, int32_t geom, int32_t storage, int64_t W, int64_t H,

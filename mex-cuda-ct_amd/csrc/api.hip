@@ -498,11 +498,16 @@ int pick_zrange(const mexct_opts* o, int geom, int64_t H) {
 // the call.
 // One choice per shape serves every batch size, so that batches of varying
 // size do not each pay for tuning.
+// The kernel is part of the key: near sources (and, cone f32, the batch) choose between
+// kernels, and the choice timed on one says nothing of another's.
+enum { KERNEL_GENERAL, KERNEL_COLUMN, KERNEL_LDS, KERNEL_COUNT };
 struct TuneKey {
   int op, geom, st;
   int64_t W, H, n;
+  int kernel;
   bool operator<(const TuneKey& o) const {
-    return std::tie(op, geom, st, W, H, n) < std::tie(o.op, o.geom, o.st, o.W, o.H, o.n);
+    return std::tie(op, geom, st, W, H, n, kernel) <
+           std::tie(o.op, o.geom, o.st, o.W, o.H, o.n, o.kernel);
   }
 };
 struct TuneVal {
@@ -861,7 +866,8 @@ int fp_run(mexct_ctx* c, const void* vol, int32_t vol_dtype, int items, int64_t 
     auto launch = [&](const FPZLaunch& l) {
       return layout == LAYOUT_COL ? launch_fpc(l, c->stream) : launch_fpz(l, c->stream);
     };
-    const TuneKey key{MEXCT_OP_FP, geom, st, W, H, nProj};
+    const TuneKey key{MEXCT_OP_FP, geom, st, W, H, nProj,
+                      layout == LAYOUT_COL ? KERNEL_COLUMN : KERNEL_GENERAL};
     TuneVal tv;
     if (tune_find(key, &tv)) {
       z.vchunk_log2 = tv.a;
@@ -1038,7 +1044,8 @@ int bp_run(mexct_ctx* c, const void* sino, int32_t sino_dtype, int items, int64_
   a.out_stride = (uint64_t)W * W * H;
   RC(upload_ptrs(c, out_ptrs, items, &a.outs));
   a.loads_only = loads_only;
-  const TuneKey key{MEXCT_OP_BP, geom, st, W, H, nProj};
+  const TuneKey key{MEXCT_OP_BP, geom, st, W, H, nProj,
+                    col ? KERNEL_COLUMN : lds ? KERNEL_LDS : KERNEL_GENERAL};
   TuneVal tv;
   const bool found = tune_find(key, &tv);
   const bool tune = !found && !loads_only && nProj > 0 && want_tune(c, key);
@@ -1153,7 +1160,9 @@ int mexct_tuned_config(int32_t op, int32_t geom, int32_t storage, int64_t W, int
                        int64_t nProj, int32_t* cfg) {
   if (!cfg) return fail(MEXCT_EINVAL, "cfg is null");
   TuneVal v;
-  const bool f = tune_find(TuneKey{op, geom, storage, W, H, nProj}, &v);
+  bool f = false;
+  for (int k = KERNEL_COUNT - 1; k >= 0 && !f; --k)
+    f = tune_find(TuneKey{op, geom, storage, W, H, nProj, k}, &v);
   cfg[0] = f ? 1 : 0;
   cfg[1] = f ? v.a : -1;
   cfg[2] = f ? v.b : -1;
