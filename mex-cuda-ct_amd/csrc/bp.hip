@@ -79,6 +79,7 @@ struct BPKArgs {
   // the z-ranges run one after another, each in a phase of phase_blocks grid
   // blocks of which the first phase_logical work
   uint32_t phase_blocks, phase_logical;
+  uint32_t group;  // blocks that an XCD takes at a time (xcd_deal)
   uint64_t sino_stride;  // bytes between the items' haloed sinograms
   uint64_t out_stride;   // floats between the items' volumes
   float* const* outs;    // non-null: item i's volume at outs[i]
@@ -177,13 +178,13 @@ template <int GEOM, int ZR, typename S, bool SMALL, int RQ, bool ZC, bool LOADS 
 __global__ __launch_bounds__(64) void bp_kernel(BPKArgs a) {
   // Block order: the z-ranges one after another over the whole chip (a
   // phase each), and in a phase (batch item, tile), the rows of super-tiles
-  // dealt to the XCDs in turn (xcd_deal).  Tiles go in super-tiles (row-major
+  // dealt to the XCDs in turn (xcd_deal; few_views).  Tiles go in super-tiles (row-major
   // inside), so that the blocks that run together cover compact regions whose
   // view footprints overlap; the voxels of one z-range project to a band of
   // detector rows whose row-paired copy stays in the memory-side cache
   // across the phase.
   const uint32_t zr = blockIdx.x / a.phase_blocks;
-  const uint32_t bl = xcd_deal(blockIdx.x - zr * a.phase_blocks, a.super_);
+  const uint32_t bl = xcd_deal(blockIdx.x - zr * a.phase_blocks, a.group);
   if (bl >= a.phase_logical) return;
   const uint32_t tiles = a.item_blocks / a.nz;
   const uint32_t item = bl / tiles;  // batch item
@@ -412,11 +413,23 @@ __global__ __launch_bounds__(64) void bp_kernel(BPKArgs a) {
 
 static unsigned padded_grid(uint32_t n_logical) { return (n_logical + 7u) & ~7u; }
 
+// Up to so many views a launch lasts as long as its stores, which run faster with a
+// contiguous range of tiles per XCD than with the tiles dealt: f16, 1 / 2 / 3 / 4 / 6 views
+// of 512^3 326 / 305 / 300 / 312 / 364 us contiguous, 372 / 367 / 361 / 329 / 345 dealt, of
+// 301^2 x 211 61 / 63 / 68 / 75 / 92 and 65 / 68 / 68 / 73 / 86; f32 near source, 1 / 2 / 3
+// views of 300^3 73 / 100 / 119 and 78 / 91 / 105.  (The column and the LDS kernel, whose
+// workgroups write more slices each, are faster dealt from one view on.)
+template <typename S>
+constexpr int few_views() {
+  return sizeof(S) == 2 ? 3 : 1;
+}
+
 template <int ZR, typename S, bool SMALL, int RQ, bool ZC>
 static void bp_dispatch_g(const BPKArgs& k0, int geom, hipStream_t st) {
   BPKArgs k = k0;  // z-ranges outermost (see bp_kernel)
   k.phase_logical = k.item_blocks / k.nz * (k.n_logical / k.item_blocks);
-  k.phase_blocks = xcd_deal_blocks(k.phase_logical, k.super_);
+  k.group = k.nviews > few_views<S>() ? k.super_ : (k.phase_logical + 7u) / 8u;
+  k.phase_blocks = xcd_deal_blocks(k.phase_logical, k.group);
   const unsigned g = k.phase_blocks * k.nz;
   if (k.loads_only) {  // cone only (the host checks)
     bp_kernel<GEOM_CONE, ZR, S, SMALL, RQ, ZC, true><<<g, 64, 0, st>>>(k);
