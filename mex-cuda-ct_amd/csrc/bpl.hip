@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256, 5) void bpl_kernel(BPLArgs a) {
     __syncthreads();
     issue(d, 0, 0, 0);
     float cn = start(0);
-    geometry(BPL_VIEWS, 1);
+    if (a.nviews > BPL_VIEWS) geometry(BPL_VIEWS, 1);
     put(d);
     __syncthreads();
     int b = 0;
@@ -198,7 +198,9 @@ __global__ __launch_bounds__(256, 5) void bpl_kernel(BPLArgs a) {
       for (int w0 = 0; w0 < BPL_VIEWS; ++w0) {
         const bool last = w0 + 1 == BPL_VIEWS;
         const float cs = cn;
-        issue(d, v + w0 + 1, last ? 0 : w0 + 1, last ? b ^ 1 : b);
+        // (past the last group, whose buffer nothing has filled: this one's again)
+        const int bn = last && v + BPL_VIEWS < a.nviews ? b ^ 1 : b;
+        issue(d, v + w0 + 1, last ? 0 : w0 + 1, bn);
         cn = start(v + w0 + 1);
         __builtin_amdgcn_sched_barrier(0);  // the next view's loads stay ahead
         if (zc > 0 && v + w0 < a.nviews) {
@@ -244,6 +246,9 @@ __global__ __launch_bounds__(256, 5) void bpl_kernel(BPLArgs a) {
             }
           }
         }
+        // a scan that ends with this view stages no more (one view of 400^3: 129 -> 111 us;
+        // the test at the group's other views too: 1.5% slower at 256^3 x 360)
+        if (w0 == 0 && v + 1 >= a.nviews) goto summed;
         __syncthreads();
         if (last) {
           geometry(v + 2 * BPL_VIEWS, b);  // the group after next, over this one
@@ -254,6 +259,7 @@ __global__ __launch_bounds__(256, 5) void bpl_kernel(BPLArgs a) {
       }
     }
   }
+summed:
   if (in_vol) {
     float* q = o;
 #pragma unroll

@@ -87,8 +87,9 @@ def record(calls, memory=None):
                        capture_output=True)
     assert r.returncode == 0, r.stderr[-3000:]
     out = json.loads(r.stdout.splitlines()[-1])
-    names = subprocess.run(["c++filt"], input=open(log).read(), text=True, capture_output=True,
-                           check=True).stdout
+    # (c++filt does not know _Float16's code, DF16_)
+    names = subprocess.run(["c++filt"], input=open(log).read().replace("DF16_", "Dh"), text=True,
+                           capture_output=True, check=True).stdout
     at = -1
     for c in out:
         c["mallocs"], c["kernels"] = [], []
