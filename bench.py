@@ -26,14 +26,25 @@ sys.path.insert(0, os.path.join(ROOT, "oracle"))  # the checker (cpu_baseline, F
 
 HBM_PEAK_GBS = 8000.0
 VC_PEAK_GBS = 256 * 64 * 2.4  # vector L1 caches: 64 B/clock per CU, 256 CUs, 2.4 GHz
+LDS_PEAK_GBS = 256 * 128 * 2.4  # LDS reads: 128 B/clock per CU
 # Memory-side bytes of one cone 384^3 x 512 f32 FP launch from rocprofv3
 # --pmc FETCH_SIZE and WRITE_SIZE (copy-calibrated): what the L2s fetched from
 # and wrote to beyond themselves (the memory-side cache or HBM).  Valid for
 # the kernel sources whose hash is stamped beside it; a changed source
 # reports null until the counters are taken again.
 FP_TRAFFIC = {"bytes": 55.57e9, "sources_sha16": "1931082f8dbf9abc"}
+
 FP_KERNEL_SOURCES = ("mex-cuda-ct_amd/csrc/fpz.hip", "mex-cuda-ct_amd/csrc/ray.h",
                      "mex-cuda-ct_amd/csrc/common.h")
+
+
+def unit_frac(kind, storage, size, rate):
+    """The gather rate (GB/s) as a fraction of the unit that the gathers go through: the
+    vector caches, or LDS, from which the f32 cone backprojection of cubes above 68^3
+    takes its taps (and each detector pixel about twenty times)."""
+    if kind == "bp" and storage == 0 and size > 68:
+        return {"frac_of_lds_peak": round(rate / LDS_PEAK_GBS, 4)}
+    return {"frac_of_vector_cache_peak": round(rate / VC_PEAK_GBS, 4)}
 
 
 def kernel_sources_sha16():
@@ -203,7 +214,7 @@ def main():
             p = nbytes / (tl * 1e-3) / 1e9
             out[k] = {"achieved_GBs": round(a, 1), "measured_peak_GBs": round(p, 1),
                       "frac": round(a / p, 4), "loads_only_ms": round(tl, 3),
-                      "frac_of_vector_cache_peak": round(a / VC_PEAK_GBS, 4)}
+                      **unit_frac(k, storage, W, a)}
         return out
 
     gather = gather_fracs(mexct.F32, fp_ms, bp_ms, vol)
@@ -214,7 +225,7 @@ def main():
                            "storage bytes each)",
                    "ceiling": "measured_peak = the operator's loads-only form (same launch, "
                               "every load, taps XOR-folded instead of interpolated)",
-                   "vector_cache_peak_GBs": VC_PEAK_GBS})
+                   "vector_cache_peak_GBs": VC_PEAK_GBS, "lds_peak_GBs": LDS_PEAK_GBS})
     log(f"[bench] gather roofline: FP {gather['fp']['achieved_GBs']:.0f}/"
         f"{gather['fp']['measured_peak_GBs']:.0f} GB/s ({gather['fp']['frac']:.2f}), "
         f"BP {gather['bp']['achieved_GBs']:.0f}/{gather['bp']['measured_peak_GBs']:.0f} GB/s "
