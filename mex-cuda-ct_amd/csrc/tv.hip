@@ -13,7 +13,10 @@
 //     instead of 20 in three, and two square roots, two reciprocals and four
 //     residual-corrected products per voxel instead of four IEEE square roots
 //     and divisions.  A step: 256^3 104 -> 58 us, 251 x 233 x 201 86 -> 43, 128^3
-//     25 -> 15, 32^3 12 -> 6.5 (launch-bound), 384^3 384 -> 265.
+//     25 -> 15, 32^3 12 -> 6.5 (launch-bound), 384^3 384 -> 250.  At 251 x 233 x 201
+//     the VALU bounds it (0.90 instructions per busy clock of a CU, the CUs busy
+//     three quarters of a step, 4.6 TB/s beyond the L2s), at 384^3 memory (4.3 TB/s,
+//     of 4.75 that a copy reaches; 0.57 VALU per clock).
 //   tv_axpy_kernel: the last step's update.
 // The launches stay on the stream: no host round trip per step.
 #include <algorithm>
@@ -191,8 +194,6 @@ __global__ __launch_bounds__(256) void tv_step_kernel(TVStep t) {
   const int kend = min(k0 + t.zc, t.nz);  // slices [k0, kend) are output
   const bool out_lane = li >= 1 && li < LW - 1 && ix < t.nx;
   const bool x_in = ix >= 1 && ix < t.nx - 1;
-  // (1 x 300 x 65000, 20 steps: 74.4 ms with the quotients that no voxel takes, 27.7 without)
-  const bool inner = t.nx > 2 && t.ny > 2 && t.nz > 2;
   const int cx = clampi(ix, 0, t.nx - 1);
   // addresses of rows y0 - 1 .. y0 + RY, clamped into the volume (a clamped
   // row's values reach no interior gradient)
@@ -249,10 +250,7 @@ __global__ __launch_bounds__(256) void tv_step_kernel(TVStep t) {
   load(k0);
 #pragma unroll
   for (int r = 0; r < RY; ++r) part[r] = 0.f;
-  // rows past the volume's are not walked (2000 x 3 x 2000, 20 steps: 2.42 -> 1.79 ms, with
-  // tv_plan's rows for so few 1.33)
-  const int klast = y0 < t.ny ? kend : k0 - 1;
-  for (int k = k0; k <= klast; ++k) {
+  for (int k = k0; k <= kend; ++k) {
     const bool odd = take(cur);
     if (k < kend) load(k + 1);
     if (k < kend && !FIRST && out_lane) {
@@ -281,12 +279,7 @@ __global__ __launch_bounds__(256) void tv_step_kernel(TVStep t) {
         }
       }
     };
-    if (!inner) {  // no voxel has a gradient: nothing to compute
-      if (k > k0 && out_lane)
-#pragma unroll
-        for (int r = 0; r < RY; ++r)
-          if (y0 + r < t.ny) t.gout[gsz * (k - 1) + ix + (size_t)t.nx * (y0 + r)] = 0.f;
-    } else if (odd || prev_odd)
+    if (odd || prev_odd)
       slice(std::false_type{});
     else
       slice(std::true_type{});
@@ -333,7 +326,7 @@ static dim3 red_grid(int nx, int ny, int nz) {
 // nearly whole lines and whose workgroups march close together (a step of
 // 200^3, 251 x 233 x 201, 320^3, 384^3 with the first rule and with this: 35, 49,
 // 192, 344 and 38, 44, 165, 271 us), unless the volume has fewer rows than most of the
-// 16 that a workgroup then walks (2000 x 8 x 2000 151 and 161 us, 2000 x 15 x 2000 265 and
+// 16 that a workgroup then walks (2000 x 3 x 2000 74 and 120 us, 2000 x 15 x 2000 265 and
 // 246).
 struct TVPlan {
   int lw, ry, zc;
@@ -415,6 +408,20 @@ hipError_t launch_tvmin(Vol3 x, const TVWork& w, const float* c_dev, float c, in
   t.gy = (uint32_t)p.gy;
   t.n = (uint32_t)np;
   if (np >= (1ull << 31)) return hipErrorInvalidValue;
+  if (x.nx < 3 || x.ny < 3 || x.nz < 3) {
+    // No interior, no gradient: the first step's a is a quotient by 0, and every voxel
+    // NaN from then on.  (1 x 300 x 65000, 20 steps: 74 ms with the step kernel, 64 with the
+    // three launches a step before it, 2.1 this way)
+    hipError_t e = launch_fill(w.g, 0.f, (size_t)x.nx * x.ny * x.nz, st);
+    if (e == hipSuccess) e = launch_fill((float*)w.partials, 0.f, 2, st);
+    if (e != hipSuccess) return e;
+    tv_scale_kernel<<<1, 256, 0, st>>>(w.partials, 1, c_dev, c, w.a_dev);
+    if (clean)
+      tv_axpy_kernel<true><<<grid, block, 0, st>>>(x, x, w.g, w.a_dev);
+    else
+      tv_axpy_kernel<false><<<grid, block, 0, st>>>(x, x, w.g, w.a_dev);
+    return hipGetLastError();
+  }
   t.np = np;
   t.c_dev = c_dev;
   t.c = c;

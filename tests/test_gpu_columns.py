@@ -118,9 +118,9 @@ def test_column_fp_compensated_sums_equal_ray_fp(gpu, monkeypatch, st):
     assert np.array_equal(out[0], out[1])
 
 
-# slices: one, a lane's 4 (8) and its neighbours, around a workgroup's 16..128;
-# columns: odd, around tiles of 8, the smallest circle; views: around the four
-# of a stage; sizes past the 2048 workgroups from which it takes 64 (128)
+# slices: one, a lane's 4 (8) and its neighbours, up to several workgroups' 32 (64);
+# columns: odd, around tiles of 8, the smallest circle; views: around a stage's.  All
+# take the fewest slices per workgroup (test_column_variants.py has the others)
 BP_SIZES = [(1, 5, 2), (3, 2, 3), (4, 1, 1), (9, 3, 5), (16, 16, 4), (33, 17, 7), (40, 65, 3), (23, 130, 9),
             (200, 131, 6), (370, 3, 2)]
 

@@ -1,6 +1,8 @@
-"""The cone f32 backprojector that gathers from LDS: bit for bit against the
-oracle at the edges of its tiles, slices per wave, windows and view groups, and
-around the sources and heights where the general kernel takes over."""
+"""Cone f32 backprojections, bit for bit against the oracle at odd sizes and around the
+sources and heights where the LDS kernel gives way to the general one: 64x64, 57x97,
+129x150, 90x192, 17x40 and 256x50 take the LDS kernel, with 16 slices per wave, the
+others (and the angle that is not finite) the general one.  Every variant of the LDS
+kernel is in test_cone_variants.py."""
 import numpy as np
 import pytest
 
@@ -9,10 +11,8 @@ import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# slices: around 64, 96 and 128 per workgroup and 16 per wave, a last workgroup
-# with one slice; columns: odd, partial tiles; views: around the four of a group;
-# sources: far, the nearest whose tiles reach 16 and 20 detector columns, and
-# nearer ones (general kernel); tall detectors, whose edge rows are read
+# slices: around 64 and 128, 16 per wave; columns: odd, partial tiles; views: around
+# the four of a group; sources: far and near; tall detectors, whose edge rows are read
 CASES = [(64, 64, 9, 1000.0), (57, 97, 6, 300.0), (33, 129, 5, 44.0), (33, 130, 4, 30.0),
          (129, 150, 3, 400.0), (200, 70, 4, 600.0), (200, 61, 3, 250.0), (24, 600, 7, 60.0),
          (90, 192, 1, 150.0), (48, 65, 13, 52.0), (17, 40, 8, 200.0), (256, 50, 2, 900.0)]

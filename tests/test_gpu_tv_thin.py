@@ -32,3 +32,17 @@ def test_thin(gpu, shape):
     got = mexct.CUDAmex_TVmin_3D(x, 0.01, steps=2)
     assert np.array_equal(got, ref, equal_nan=True)
     assert np.isnan(got).all() == (min(shape) < 3)
+
+
+@pytest.mark.gpu
+def test_thin_osc_tv(gpu):
+    # the reconstruction's TV steps of a volume of two columns: NaN, which it zeroes
+    r = np.random.Generator(np.random.PCG64(2))
+    W, H, n = 2, 9, 6
+    pre = np.asfortranarray(r.uniform(0.9e4, 1.1e4, (W, H, n)).astype(np.float32))
+    post = np.asfortranarray((pre * r.uniform(0.5, 0.9, pre.shape)).astype(np.float32))
+    ang = (np.arange(n) * 1.0).astype(np.float32)
+    for geom in ("par3d", "cone3d"):
+        got = mexct.OSC_TV_recon(pre, post, ang, {"type": geom, "SAD": 100.0}, 3, 0.1, 2, 1, 1.0,
+                                 tv_steps=3, picks=np.ones(3, np.int32))
+        assert np.array_equal(got, np.zeros((W, W, H), np.float32)), geom
