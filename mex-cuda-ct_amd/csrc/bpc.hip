@@ -23,13 +23,13 @@
 //
 // What bounds it: the LDS reads, 8 bytes (f32) or 4 (2-byte) an update and 2 or
 // 1 of geometry, at 128 bytes per clock per CU; 384^3 x 512 par f32 runs at
-// about 0.65 of that.  With the copy, the general kernel -> columns: 128^3 x 180
-// views par f32 390 -> 103 us, f16 280 -> 111; 256^3 x 360 par f32 3.11 -> 0.93
-// ms, fan f32 3.13 -> 1.09, f16 2.07 -> 0.73, bf16 2.41 -> 0.89; 384^3 x 512 par
-// f32 13.2 -> 4.4 ms, fan f16 8.2 -> 3.4.  (One scalar geometry per wave, 64
-// lanes along z, read by v_readlane: 5.3 ms at 384^3 f32, its registers and the
-// idle rows past H cost more than the broadcast reads save; four waves, no
-// prefetch, three barriers a stage: 7.0 ms.)
+// 0.77 of that.  The call, general kernel -> columns: 128^3 x 180 views par f32
+// 393 -> 110 us, f16 280 -> 114; 256^3 x 360 par f32 3.08 -> 0.85 ms, fan f32 3.11 ->
+// 1.01, par f16 2.00 -> 0.70, bf16 2.30 -> 0.82; 384^3 x 512 par f32 13.0 -> 3.71 ms, fan
+// f16 8.05 -> 2.95.  (Before the tiles were dealt to the XCDs, at 384^3 par f32 4.4 ms:
+// one scalar geometry per wave, 64 lanes along z, read by v_readlane, 5.3 ms, its
+// registers and the idle rows past H cost more than the broadcast reads save; four
+// waves, no prefetch, three barriers a stage, 7.0 ms.)
 //
 // The reference's row lerp fma(0, c1 - c0, c0) returns c0 where the taps of
 // row z + 1 are finite and NaN where one is not; the copy holds NaN where the

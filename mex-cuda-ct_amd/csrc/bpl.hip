@@ -10,9 +10,10 @@
 // 13 VALU per update, no row clamp (the copy has a halo of edge rows).  Bound by
 // LDS (89% busy at 384^3, 5.2 clocks for each 8-byte read of a wave, 4 at least)
 // and next the VALU (14.7 instructions an update with set-up).
-// Against the general kernel: 384^3 x 512 views 15.3 -> 11.6 ms, 256^3 x 360 3.90 ->
-// 2.38, 301^2 x 211 x 250 3.29 -> 2.35, 64^3 x 60 169 -> 98 us; never slower from 32^3
-// to 512^2 x 400 (with the tiles dealt to the XCDs, xcd_deal, 9.5, 2.2 and 2.0 ms).
+// The call, general kernel (with contiguous tiles per XCD) -> this one: 384^3 x 512
+// views 15.2 -> 9.6 ms, 256^3 x 360 3.87 -> 2.20, 301^2 x 211 x 250 3.33 -> 1.96, 128^3 x
+// 180 503 -> 291 us, 64^3 x 60 173 -> 99.  Slower only for one or two views of 350^2 to
+// 450^2 (one of 450^2 x 300: 114 -> 137 us).  The scans it does not take: see bpl_plan.
 //
 // A 256-thread workgroup: wave w sums slices [w ZR, (w+1) ZR) of its 4 ZR, one
 // voxel column per lane, sums in registers over the views in the reference's
@@ -271,7 +272,11 @@ summed:
 }
 
 // The launch for a cone scan: slices per wave, the window and the copy's rows;
-// false where the general kernel is taken.
+// false where the general kernel is taken: W < 4 or > 4096, more than 2048 rows,
+// sources within 20% of the circle or whose tiles reach more than 20 detector
+// columns, and scans whose cheapest slice count would need a larger copy than the
+// general kernel's (half of those below 68^2, 5% of the others up to 512^2: 33^2 x 32 at
+// SAD 500 and 32^3, 130^2 x 70 at 553, 221^2 x 120 at 618).
 struct BPLPlan {
   int zr, p, cw, rw, zt, pv;
   double umax;

@@ -34,7 +34,8 @@ hipError_t launch_pad3z(const void* in, int in_dt, int64_t in_sy, int64_t in_sz,
 // rows 30.8, 30.9, 31.2 and 31.3 ms at 504 to 516.  Other rows stay as tight as
 // they are: whole odd numbers of lines ran the general-3D projection 9% slower.
 // The dual copy, of which a sample loads two rows, takes rows of 48 or 80 bytes
-// past a multiple of 128, the best of 12 rows tried at six sizes: cone 384^3 x 512
+// past a multiple of 128, the best of 12 rows tried at six sizes (measured; no counter
+// says why): cone 384^3 x 512
 // views 25.6 -> 24.5 ms, 256^3 x 360 5.27 -> 5.11, general-3D 320^3 x 360 22.2 ->
 // 21.4, 250^2 x 187 x 240 8.70 -> 8.04; the quads show no such order.
 inline int64_t fp_zrow(int64_t n, int64_t nz, bool dual) {
